@@ -64,6 +64,9 @@ int ensure_pattern(Ctx *c) {
     tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
     adj.insert(adj.end(), tmp.begin(), tmp.end());
     adj_off[i + 1] = (long long)adj.size();
+    c->max_deg = std::max(c->max_deg, (int)tmp.size());
+    if (!tmp.empty())
+      c->bandwidth = std::max({c->bandwidth, (int)i - tmp.front(), tmp.back() - (int)i});
   }
   // CSR rows: node-major, P rows per node, each with P*deg columns (neighbour m, comp d) sorted
   c->h_row_ptr.assign(c->Ndof + 1, 0);

@@ -106,6 +106,8 @@ struct Ctx {
   int *d_col_idx = nullptr;
   uint8_t *d_slot = nullptr;  // (Ne*n*n) position of node b in node a's sorted neighbour list
   int *d_diag_off = nullptr;  // (Ndof) offset of the diagonal entry within each CSR row
+  int max_deg = 0;            // most neighbours of a node, itself included
+  int bandwidth = 0;          // largest |m - i| over neighbours m of nodes i
   int *d_ne_off = nullptr;    // (Nn+1) node -> incident (element, local index) entries
   int *d_ne_list = nullptr;   // (Ne*n) element * n + local index, element order within a node
   bool have_colour = false;

@@ -15,7 +15,7 @@
 // the FP32 solves in FP64 iterative refinement r = b - A x with the FP64 matrix.
 #include <cmath>
 
-#include "femhot_kernels.h"
+#include "femhot_pcg_tile.h"
 
 namespace femhot {
 
@@ -398,14 +398,163 @@ static int pcg_core(Ctx *c, long long n, const long long *rp, const int *ci, con
   return FEMHOT_OK;
 }
 
-// State of a device-side-stopped PCG (femhot_pcg_async): status 0 running, 1 converged, 2 non-finite
-// residual, 3 iteration budget spent.  Every guarded kernel returns at once when status != 0.
-struct PcgState {
-  int status;
-  int iters;
-  double bnorm2;
-  double rr;
+// How a system is cut for the tile kernels: G workgroups of 512 threads, `lpn` lanes per node, S nodes per
+// group of lanes.  ok only on the context's pattern, for systems whose rows fit: at most 4 neighbour
+// blocks per lane, the S x 4 blocks of a lane within the register file, one workgroup per CU, a
+// workgroup's columns within TILE_RANGE ids and its vectors within LDS.
+struct TilePlan {
+  bool ok = false;
+  int lpn = 4, S = 1, G = 0, cap = 0;
+  size_t lds = 0;
 };
+
+static int device_cus() {
+  static int cus = 0;
+  if (!cus) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      cus = 256;
+  }
+  return cus;
+}
+
+// Most nodes per lane group: S x 4 x P x P values of T within about 150 registers.
+template <class T> constexpr int tile_max_s(int P) { return P == 1 ? 8 : P == 2 ? 4 : sizeof(T) == 4 ? 4 : 2; }
+
+// Calls f(integral_constant P, LPN, S) for a plan (S within what tile_plan chooses for P and T).
+template <class T, class F> static int tile_dispatch(int P, const TilePlan &tp, F &&f) {
+  using std::integral_constant;
+  auto with_s = [&](auto p, auto l) -> int {
+    constexpr int MAXS = tile_max_s<T>(decltype(p)::value);
+    if constexpr (MAXS >= 8)
+      if (tp.S == 8) return f(p, l, integral_constant<int, 8>{});
+    if constexpr (MAXS >= 4)
+      if (tp.S == 4) return f(p, l, integral_constant<int, 4>{});
+    if constexpr (MAXS >= 2)
+      if (tp.S == 2) return f(p, l, integral_constant<int, 2>{});
+    return f(p, l, integral_constant<int, 1>{});
+  };
+  auto with_l = [&](auto p) -> int {
+    return tp.lpn == 4 ? with_s(p, integral_constant<int, 4>{}) : with_s(p, integral_constant<int, 8>{});
+  };
+  if (P == 1) return with_l(integral_constant<int, 1>{});
+  if (P == 2) return with_l(integral_constant<int, 2>{});
+  return with_l(integral_constant<int, 3>{});
+}
+
+template <class T> static TilePlan tile_plan(const Ctx *c) {
+  TilePlan tp;
+  if (c->max_deg < 1 || c->max_deg > 8 * TILE_U) return tp;
+  tp.lpn = c->max_deg <= 4 * TILE_U ? 4 : 8;
+  const int P = c->ndpn, npw = TILE_T / tp.lpn;
+  const int max_s = tile_max_s<T>(P);
+  const int most = std::min(device_cus(), 256);
+  auto groups = [&](int s) { return (c->Nn + (long long)npw * s - 1) / ((long long)npw * s); };
+  if (groups(max_s) > most) return tp;
+  // One workgroup needs no exchange, and is taken while its passes stay few (quads 20 x 20 conduction in FP64:
+  // 2.6 us an iteration with S = 4 in one workgroup, 4.0 in four with S = 1; 40 x 40: 5.5 with S = 8 in two,
+  // 4.0 with S = 2 in seven).  Otherwise few workgroups, but not at the cost of passes where a node's block is
+  // large: from S = 1 (3 dofs per node) or 2 up to the first S that leaves at most 128 workgroups (quads
+  // 128 x 128: 7.4 us with 130, 6.1 with 65; tetrahedra 20^3 mixed: 6.1 with S = 1, 7.7 with S = 4), else up
+  // to the first that fits the device.
+  int s = P == 3 ? 1 : 2;
+  if (groups(std::min(4, max_s)) == 1) {
+    s = 1;
+    while (groups(s) > 1) s *= 2;
+  } else {
+    if (P == 1)
+      while (s < max_s && groups(s) > 128) s *= 2;
+    while (groups(s) > most) s *= 2;
+  }
+  tp.S = s;
+  tp.G = (int)groups(s);
+  const long long range = std::min<long long>(c->Nn, (long long)npw * s + 2LL * c->bandwidth);
+  if (range > TILE_RANGE) return tp;
+  tp.cap = (int)std::min<long long>(range, (long long)TILE_T * TILE_U * s);
+  tile_dispatch<T>(P, tp, [&](auto p, auto l, auto sc) {
+    tp.lds = Tile<T, decltype(p)::value, decltype(l)::value, decltype(sc)::value>::lds(tp.cap);
+    return 0;
+  });
+  static size_t lim = 0;
+  if (!lim) {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || v <= 0)
+      v = 64 * 1024;
+    lim = (size_t)v - 2048;  // less the kernel's static LDS
+  }
+  tp.ok = tp.lds <= lim;
+  return tp;
+}
+
+static size_t r256(size_t b) { return (b + 255) & ~size_t(255); }
+template <class T> static size_t tile_ws_bytes(const Ctx *c, const TilePlan &tp) {
+  return 2 * r256(sizeof(T) * c->Ndof) + r256(sizeof(double) * 8 * tp.G) + 2 * r256(sizeof(PcgState));
+}
+
+// One resident solve (k_pcg_resident), synchronised: *st the final state; *ran false when it could not be
+// launched or a wait between its workgroups ran out (x is then untouched).
+template <class T>
+static int tile_solve(Ctx *c, const TilePlan &tp, void *ws, const long long *rp, const int *ci, const double *vals,
+                      const double *b, T *x, double bnorm, double tol, int maxiter, int check, hipStream_t s,
+                      PcgState *st, bool *ran) {
+  char *w = (char *)ws;
+  auto take = [&](size_t bytes) {
+    char *p = w;
+    w += r256(bytes);
+    return (void *)p;
+  };
+  TileArgs A{};
+  A.nodes = c->Nn;
+  A.rp = rp;
+  A.ci = ci;
+  A.vals = vals;
+  A.doff = c->d_diag_off;
+  A.b = b;
+  A.x = x;
+  A.z[0] = take(sizeof(T) * c->Ndof);
+  A.z[1] = take(sizeof(T) * c->Ndof);
+  A.pa = (double *)take(sizeof(double) * 8 * tp.G);
+  A.pc = A.pa + 6 * tp.G;
+  A.st = (PcgState *)take(sizeof(PcgState));
+  A.fail = (int *)(A.st + 1);
+  (void)take(sizeof(PcgState));
+  A.G = tp.G;
+  A.bw = c->bandwidth;
+  A.cap = tp.cap;
+  A.bnorm = bnorm;
+  A.tol = tol;
+  A.maxiter = maxiter;
+  A.check = check;
+  const long long nc = std::max<long long>(c->Ndof, 8LL * tp.G);
+  hipLaunchKernelGGL((k_tile_clear<T>), dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, A, c->Ndof);
+  *ran = false;
+  int rc = tile_dispatch<T>(c->ndpn, tp, [&](auto p, auto l, auto sc) -> int {
+    auto k = k_pcg_resident<T, decltype(p)::value, decltype(l)::value, decltype(sc)::value>;
+    if (tp.G == 1) {
+      hipLaunchKernelGGL(k, dim3(1), dim3(TILE_T), tp.lds, s, A);
+      *ran = hipGetLastError() == hipSuccess;
+    } else {
+      // cooperative: the runtime starts it only with every workgroup resident
+      void *args[] = {&A};
+      *ran = hipLaunchCooperativeKernel((const void *)k, dim3(tp.G), dim3(TILE_T), args, (unsigned)tp.lds, s) == hipSuccess;
+      (void)hipGetLastError();
+    }
+    return FEMHOT_OK;
+  });
+  if (rc || !*ran) return rc;
+  struct Out {
+    PcgState st;
+    int fail;
+  };
+  Out *o = (Out *)c->h_pinned;
+  FH_HIP(hipMemcpyAsync(o, A.st, sizeof(PcgState) + sizeof(int), hipMemcpyDeviceToHost, s));
+  FH_HIP(hipStreamSynchronize(s));
+  *ran = !o->fail && o->st.status != 0;
+  *st = o->st;
+  return FEMHOT_OK;
+}
 
 // Sum (fixed order) of NBR partials by one workgroup of 1024 threads.
 __device__ __forceinline__ double sum_nbr_1024(const double *part) {
@@ -518,14 +667,42 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
   const size_t nsp = sp.blocks;
   size_t need = (4 * NBR + nsp + 8) * sizeof(double) + 1024 + 5 * vec64 + 1024;
   if (mode == FEMHOT_F32) need += 5 * vec32 + sizeof(float) * nnz + 1024;
+  // systems the tile kernels hold are solved in one launch (mixed: one launch per inner solve)
+  TilePlan tp;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  FH_HIP(hipStreamIsCapturing(s, &cs));
+  if (node_blocked && cs == hipStreamCaptureStatusNone)
+    tp = mode == FEMHOT_F64 ? tile_plan<double>(c) : tile_plan<float>(c);
+  const size_t tile_bytes = !tp.ok ? 0 : mode == FEMHOT_F64 ? tile_ws_bytes<double>(c, tp) : tile_ws_bytes<float>(c, tp);
+  need = std::max(need, tile_bytes) + (mode == FEMHOT_F32 ? tile_bytes : 0);
   rc = ensure_workspace(c, need);
   if (rc) return rc;
+  if (tp.ok && mode == FEMHOT_F64) {
+    PcgState st{};
+    bool ran = false;
+    rc = tile_solve<double>(c, tp, c->d_ws, row_ptr, col_idx, vals, b, x, -1.0, tol, maxiter, check, s, &st, &ran);
+    if (rc) return rc;
+    if (ran) {
+      if (iters) *iters = st.iters;
+      if (st.status == 2) {
+        set_error("femhot_pcg: non-finite residual");
+        return FEMHOT_ERR_NONFINITE;
+      }
+      if (rel_res) *rel_res = st.bnorm2 > 0.0 ? std::sqrt(std::max(st.rr, 0.0) / st.bnorm2) : 0.0;
+      if (st.status != 1) {
+        set_error("femhot_pcg: maximum iterations reached");
+        return FEMHOT_ERR_NOT_CONVERGED;
+      }
+      return FEMHOT_OK;
+    }
+  }
   char *ws = (char *)c->d_ws;
   auto take = [&](size_t bytes) {
     char *p = ws;
     ws += (bytes + 255) & ~size_t(255);
     return (void *)p;
   };
+  void *tile_ws = mode == FEMHOT_F32 && tp.ok ? take(tile_bytes) : nullptr;
   double *sc = (double *)take(3 * NBR * sizeof(double));
   double *aux = (double *)take(NBR * sizeof(double));
   double *pap_part = (double *)take(nsp * sizeof(double));
@@ -553,12 +730,17 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
     float *v32 = (float *)take(sizeof(float) * nnz);
     float *x32 = (float *)take(vec32), *r32 = (float *)take(vec32), *p32 = (float *)take(vec32);
     float *q32 = (float *)take(vec32), *dinv32 = (float *)take(vec32);
-    const unsigned cg = (unsigned)std::min<long long>((nnz + 255) / 256, 65536);
-    hipLaunchKernelGGL((k_cast<float>), dim3(cg), dim3(256), 0, s, nnz, vals, v32);
-    if (node_blocked)
-      hipLaunchKernelGGL((k_diag_inv_pos<float>), grid, dim3(256), 0, s, n, row_ptr, c->d_diag_off, vals, dinv32);
-    else
-      hipLaunchKernelGGL((k_diag_inv<float>), grid, dim3(256), 0, s, n, row_ptr, col_idx, vals, dinv32);
+    bool cast_done = false;
+    auto cast = [&] {  // the FP32 matrix and diagonal of the launched kernels (the tile kernels convert as they load)
+      if (cast_done) return;
+      cast_done = true;
+      const unsigned cg = (unsigned)std::min<long long>((nnz + 255) / 256, 65536);
+      hipLaunchKernelGGL((k_cast<float>), dim3(cg), dim3(256), 0, s, nnz, vals, v32);
+      if (node_blocked)
+        hipLaunchKernelGGL((k_diag_inv_pos<float>), grid, dim3(256), 0, s, n, row_ptr, c->d_diag_off, vals, dinv32);
+      else
+        hipLaunchKernelGGL((k_diag_inv<float>), grid, dim3(256), 0, s, n, row_ptr, col_idx, vals, dinv32);
+    };
     // outer FP64 refinement: r = b - A x; solve A d = r in FP32 to inner_tol; x += d
     const double inner_tol = 1e-4;
     int outer = 0;
@@ -583,9 +765,25 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
       double rel_in = 0.0;
       bool cin = false;
       // inner solve on the FP64 residual r64 (FP32 iterates, FP64 dot products)
-      rc = pcg_core<float>(c, n, row_ptr, col_idx, v32, r64, x32, r32, p32, q32, dinv32, sc, pap_part, pap, bnorm * rel,
-                           std::max(inner_tol, 0.5 * tol / std::max(rel, 1e-300)), maxiter - it, check, sp, s,
-                           &k_in, &rel_in, &cin);
+      const double tol_in = std::max(inner_tol, 0.5 * tol / std::max(rel, 1e-300));
+      bool ran = false;
+      if (tile_ws) {
+        PcgState st{};
+        rc = tile_solve<float>(c, tp, tile_ws, row_ptr, col_idx, vals, r64, x32, bnorm * rel, tol_in, maxiter - it,
+                               check, s, &st, &ran);
+        if (rc) return rc;
+        k_in = st.iters;
+        if (ran && st.status == 2) {
+          set_error("femhot_pcg: non-finite residual");
+          if (iters) *iters = it + k_in;
+          return FEMHOT_ERR_NONFINITE;
+        }
+        if (!ran) tile_ws = nullptr;
+      }
+      if (!ran) cast();
+      if (!ran)
+        rc = pcg_core<float>(c, n, row_ptr, col_idx, v32, r64, x32, r32, p32, q32, dinv32, sc, pap_part, pap, bnorm * rel,
+                             tol_in, maxiter - it, check, sp, s, &k_in, &rel_in, &cin);
       if (rc) return rc;
       it += std::max(k_in, 1);
       hipLaunchKernelGGL((k_axpy_to64<float>), grid, dim3(256), 0, s, n, x32, x);
@@ -605,7 +803,10 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
 // Workspace of femhot_pcg_async: the layout of femhot_pcg in FP64 mode plus the solver state, each piece
 // 256-byte aligned.
 static size_t pcg_async_ws_bytes(const Ctx *c, bool node_blocked) {
-  auto r256 = [](size_t b) { return (b + 255) & ~size_t(255); };
+  if (node_blocked) {
+    const TilePlan tp = tile_plan<double>(c);
+    if (tp.ok) return 6 * r256(sizeof(double) * c->Ndof) + r256(sizeof(double) * 8 * tp.G) + r256(sizeof(PcgState));
+  }
   const size_t vec64 = sizeof(double) * c->Ndof;
   const size_t nsp = spmv_plan(c->Ndof, c->nnz, c->ndpn, node_blocked).blocks;
   return r256(3 * NBR * sizeof(double)) + r256(NBR * sizeof(double)) + r256(nsp * sizeof(double)) +
@@ -660,6 +861,47 @@ static int pcg_async_core(Ctx *c, bool node_blocked, const long long *row_ptr, c
     ws += (bytes + 255) & ~size_t(255);
     return (void *)p;
   };
+  const TilePlan tp = node_blocked ? tile_plan<double>(c) : TilePlan{};
+  if (tp.ok) {  // the phases of the resident solve, one launch each: its bits, and a graph can hold them
+    TileVecs V;
+    V.r = (double *)take(vec64);
+    V.z = (double *)take(vec64);
+    V.dinv = (double *)take(vec64);
+    V.q = (double *)take(vec64);
+    V.p[0] = (double *)take(vec64);
+    V.p[1] = (double *)take(vec64);
+    TileArgs A{};
+    A.nodes = c->Nn;
+    A.rp = row_ptr;
+    A.ci = col_idx;
+    A.vals = vals;
+    A.doff = c->d_diag_off;
+    A.b = b;
+    A.x = x;
+    A.pa = (double *)take(sizeof(double) * 8 * tp.G);
+    A.pc = A.pa + 6 * tp.G;
+    A.st = (PcgState *)take(sizeof(PcgState));
+    A.G = tp.G;
+    A.tol = tol;
+    A.maxiter = iterations;
+    int rc = tile_dispatch<double>(c->ndpn, tp, [&](auto p, auto l, auto sc) -> int {
+      constexpr int P = decltype(p)::value, LPN = decltype(l)::value, S = decltype(sc)::value;
+      const dim3 g(tp.G), t(TILE_T);
+      hipLaunchKernelGGL((k_tile_init<P, LPN, S>), g, t, 0, s, A, V);
+      hipLaunchKernelGGL(k_tile_test, dim3(1), t, 0, s, A, 0, 1, outer);
+      for (int k = 0; k < iterations; ++k) {
+        const int par = k & 1;
+        hipLaunchKernelGGL((k_tile_spmv<P, LPN, S>), g, t, 0, s, A, V, par, k == 0 ? 1 : 0);
+        hipLaunchKernelGGL((k_tile_update<P, LPN, S>), g, t, 0, s, A, V, par);
+        hipLaunchKernelGGL(k_tile_test, dim3(1), t, 0, s, A, 1 - par, 0, (const int *)nullptr);
+      }
+      hipLaunchKernelGGL(k_pcg_finish, dim3(1), dim3(64), 0, s, A.st, iters, rel_res, status);
+      FH_HIP(hipGetLastError());
+      return FEMHOT_OK;
+    });
+    if (state_out) *state_out = A.st;
+    return rc;
+  }
   double *sc = (double *)take(3 * NBR * sizeof(double));
   double *aux = (double *)take(NBR * sizeof(double));
   double *pap_part = (double *)take(nsp * sizeof(double));
