@@ -38,7 +38,8 @@ EXPORTED = [
     "femhot_energy_grad", "femhot_pcg", "femhot_spmv", "femhot_orient_elements", "femhot_autotune",
     "femhot_kernel_timing", "femhot_set_chunk_config", "femhot_residual_shape_vjp", "femhot_newton",
     "femhot_gauss_point_data", "femhot_energy_grad_noalloc", "femhot_pcg_async", "femhot_newton_async",
-    "femhot_chunk_plan_check",
+    "femhot_chunk_plan_check", "femhot_residual_vjp_scaled", "femhot_batch_residual_norm", "femhot_batch_loss",
+    "femhot_scale",
 ]
 
 OP_RESIDUAL, OP_VJP, OP_ENERGY_GRAD, OP_TANGENT = 0, 1, 2, 3
@@ -103,6 +104,10 @@ def lib():
     L.femhot_residual.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, ll, vp, u32, vp]
     L.femhot_tangent_csr.argtypes = [vp, i32, vp, vp, vp, vp, u32, vp]
     L.femhot_residual_vjp.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, ll, vp, ll, vp, ll, u32, vp]
+    L.femhot_residual_vjp_scaled.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, ll, vp, vp, ll, vp, ll, u32, vp]
+    L.femhot_batch_residual_norm.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, vp, vp, vp, u32, vp]
+    L.femhot_batch_loss.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, vp, vp, vp, vp, vp, u32, vp]
+    L.femhot_scale.argtypes = [i32, ll, vp, vp, dbl, vp, vp]
     L.femhot_energy_grad.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, vp, ll, vp, ll, u32, vp]
     L.femhot_energy_grad_noalloc.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, vp, ll, vp, ll, u32, vp]
     L.femhot_residual_shape_vjp.argtypes = [vp, i32, vp, vp, vp, vp, u32, vp]

@@ -153,8 +153,50 @@ class FemhotContext:
                                           self.n_dofs, _ptr(en), flags, _stream()))
         return R, (en.view(B, self.n_segments) if en is not None else None)
 
-    def residual_vjp(self, field, u, w, want_gu=True, want_gd=True, flags=0, out=None):
-        """(dR/du)^T w and (dR/dfield)^T w; out: preallocated contiguous (g_u, g_field) to write."""
+    def batch_residual_norm(self, field, u, flags=0):
+        """(loss, full, R) of a batch: u (B, n_dofs) with the Dirichlet dofs at their values, its masked
+        residual, and 1/2 sum R^2 as a 0-dim tensor (femhot_batch_residual_norm)."""
+        B, dt, dev = u.shape[0], u.dtype, u.device
+        us = self._check_in(u, "u", self.n_dofs, B, dt, dev)
+        fs = self._check_in(field, "field", self._field_size(flags), B, dt, dev)
+        full = torch.empty(2, B, self.n_dofs, dtype=dt, device=dev)
+        loss = torch.empty((), dtype=dt, device=dev)
+        scratch = torch.empty(256, dtype=torch.float64, device=dev)
+        at = full.data_ptr()
+        L.check(self._lib.femhot_batch_residual_norm(
+            self._h, _dtype_code(u), B, field.data_ptr(), fs, u.data_ptr(), us, at,
+            at + B * self.n_dofs * full.element_size(), loss.data_ptr(), scratch.data_ptr(), flags, _stream()))
+        return loss, full[0], full[1]
+
+    def batch_loss(self, field, u, want_R=True, flags=0):
+        """(mean, low, high, energies, full, R) of a batch (femhot_batch_loss): 0-dim statistics of the
+        samples' energies, the energies (B, n_segments) in float64, u with the Dirichlet dofs at their
+        values, and the masked residual or None."""
+        B, dt, dev = u.shape[0], u.dtype, u.device
+        us = self._check_in(u, "u", self.n_dofs, B, dt, dev)
+        fs = self._check_in(field, "field", self._field_size(flags), B, dt, dev)
+        full = torch.empty(B, self.n_dofs, dtype=dt, device=dev)
+        R = torch.empty(B, self.n_dofs, dtype=dt, device=dev) if want_R else None
+        en = torch.empty(B, self.n_segments, dtype=torch.float64, device=dev)
+        mean, low, high = (torch.empty((), dtype=dt, device=dev) for _ in range(3))
+        L.check(self._lib.femhot_batch_loss(
+            self._h, _dtype_code(u), B, field.data_ptr(), fs, u.data_ptr(), us, full.data_ptr(),
+            R.data_ptr() if want_R else None, en.data_ptr(), mean.data_ptr(), low.data_ptr(), high.data_ptr(), flags,
+            _stream()))
+        return mean, low, high, en, full, R
+
+    def scale(self, src, g, factor=1.0):
+        """src * (factor * g) for a 0-dim device tensor g of src's dtype (femhot_scale)."""
+        if not src.is_contiguous() or g.dtype != src.dtype or g.numel() != 1 or g.device != src.device:
+            raise ValueError("scale: a contiguous tensor and a one-element factor of its dtype and device")
+        out = torch.empty_like(src)
+        L.check(self._lib.femhot_scale(_dtype_code(src), src.numel(), src.data_ptr(), g.data_ptr(), float(factor),
+                                       out.data_ptr(), _stream()))
+        return out
+
+    def residual_vjp(self, field, u, w, want_gu=True, want_gd=True, flags=0, out=None, scale=None):
+        """(dR/du)^T w and (dR/dfield)^T w; out: preallocated contiguous (g_u, g_field) to write.  scale: a
+        one-element device tensor of u's dtype that multiplies w."""
         u = u if u.dim() == 2 else u.unsqueeze(0)
         w = w if w.dim() == 2 else w.unsqueeze(0)
         field = field if field.dim() == 2 else field.unsqueeze(0)
@@ -174,8 +216,11 @@ class FemhotContext:
         else:
             gu = torch.empty(B, self.n_dofs, dtype=dt, device=dev) if want_gu else None
             gd = torch.empty(B, fsz, dtype=dt, device=dev) if want_gd else None
-        L.check(self._lib.femhot_residual_vjp(self._h, _dtype_code(u), B, _ptr(field), fs, _ptr(u), us, _ptr(w), ws,
-                                              _ptr(gu), self.n_dofs, _ptr(gd), fsz, flags, _stream()))
+        if scale is not None and (scale.dtype != dt or scale.device != dev or scale.numel() != 1):
+            raise ValueError("scale must be one value of u's dtype on u's device")
+        L.check(self._lib.femhot_residual_vjp_scaled(self._h, _dtype_code(u), B, _ptr(field), fs, _ptr(u), us, _ptr(w),
+                                                     ws, _ptr(scale), _ptr(gu), self.n_dofs, _ptr(gd), fsz, flags,
+                                                     _stream()))
         return gu, gd
 
     def energy_grad(self, field, u, want_gu=True, want_gd=True, want_energy=True, flags=0, out=None):

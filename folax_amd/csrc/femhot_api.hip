@@ -32,6 +32,7 @@ struct CallIO {
   long long us = 0;
   const void *w = nullptr;
   long long ws = 0;
+  const void *wscale = nullptr;
   void *ou = nullptr;
   long long ous = 0;
   void *od = nullptr;
@@ -91,7 +92,7 @@ static int run_elem(Ctx *c, const CallIO &io_in) {
     return rc;
   if (chunk) {
     return run_chunk(c, io.dtype, io.mode, io.batch, io.field, io.fs, io.u, io.us, io.w, io.ws, io.ou, io.ous, io.od,
-                     io.ods, io.energy, io.flags, io.stream, 0, 0);
+                     io.ods, io.energy, io.flags, io.stream, 0, 0, io.wscale);
   }
   ElemLaunch L{};
   L.dtype = io.dtype;
@@ -110,6 +111,7 @@ static int run_elem(Ctx *c, const CallIO &io_in) {
   A.ustride = io.batch > 1 ? io.us : 0;
   A.w = io.w;
   A.wstride = io.batch > 1 ? io.ws : 0;
+  A.wscale = io.wscale;
   A.out_u = io.ou;
   A.oustride = io.batch > 1 ? io.ous : 0;
   A.out_d = io.od;
@@ -172,6 +174,13 @@ int femhot_residual(femhot_ctx *h, int dtype, int batch, const void *field, long
 int femhot_residual_vjp(femhot_ctx *h, int dtype, int batch, const void *field, long long fs, const void *u,
                         long long us, const void *w, long long ws, void *g_u, long long gus, void *g_field,
                         long long gfs, unsigned flags, void *stream) {
+  return femhot_residual_vjp_scaled(h, dtype, batch, field, fs, u, us, w, ws, nullptr, g_u, gus, g_field, gfs, flags,
+                                    stream);
+}
+
+int femhot_residual_vjp_scaled(femhot_ctx *h, int dtype, int batch, const void *field, long long fs, const void *u,
+                               long long us, const void *w, long long ws, const void *scale, void *g_u, long long gus,
+                               void *g_field, long long gfs, unsigned flags, void *stream) {
   FH_CHECK_ARG(h, FEMHOT_ERR_ARG, "null context");
   FH_CHECK_ARG(w, FEMHOT_ERR_ARG, "femhot_residual_vjp: null cotangent");
   CallIO io;
@@ -184,6 +193,7 @@ int femhot_residual_vjp(femhot_ctx *h, int dtype, int batch, const void *field, 
   io.us = us;
   io.w = w;
   io.ws = ws;
+  io.wscale = scale;
   io.ou = g_u;
   io.ous = gus;
   io.od = g_field;

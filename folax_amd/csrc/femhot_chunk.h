@@ -5,10 +5,11 @@
 namespace femhot {
 
 // Runs MODE_RES / MODE_VJP / MODE_EGRAD over the chunk plan of `epc` elements per chunk
-// (0 = autotuned default) with `block` threads per workgroup (0 = default).
+// (0 = autotuned default) with `block` threads per workgroup (0 = default).  wscale: a device scalar
+// that multiplies w, or null.
 int run_chunk(Ctx *c, int dtype, int mode, int batch, const void *field, long long fs, const void *u, long long us,
               const void *w, long long ws, void *ou, long long ous, void *od, long long ods, double *energy,
-              unsigned flags, hipStream_t stream, int epc, int block);
+              unsigned flags, hipStream_t stream, int epc, int block, const void *wscale = nullptr);
 
 // Times chunk configurations (elements per chunk x workgroup size x grid shape) on the given
 // inputs with HIP events and records the fastest for (ctx, mode, dtype, batch, field location).

@@ -194,8 +194,9 @@ static size_t lds_limit() {
 // must already be built, nothing is allocated and no timing events are recorded.
 static int run_chunk_cfg(Ctx *c, int dtype, int mode, int batch, const void *field, long long fs, const void *u,
                          long long us, const void *w, long long ws, void *ou, long long ous, void *od, long long ods,
-                         double *energy, unsigned flags, hipStream_t s, const ChunkConfig &cfg,
-                         void *fixed_ws = nullptr, size_t fixed_bytes = 0) {
+                         double *energy, unsigned flags, hipStream_t s, ChunkConfig cfg,
+                         void *fixed_ws = nullptr, size_t fixed_bytes = 0, const void *wscale = nullptr) {
+  if (wscale) cfg.dma = false;  // the LDS-DMA kernel brings the cotangent to LDS as it is
   const ChunkPlan *plan = nullptr;
   int rc;
   if (fixed_ws) {
@@ -322,6 +323,7 @@ static int run_chunk_cfg(Ctx *c, int dtype, int mode, int batch, const void *fie
   A.us = batch > 1 ? us : 0;
   A.w = w;
   A.ws = batch > 1 ? ws : 0;
+  A.wscale = wscale;
   A.ou = ou;
   A.ous = batch > 1 ? ous : c->Ndof;
   A.od = mode == MODE_RES ? nullptr : od;
@@ -413,7 +415,7 @@ static ChunkConfig default_config(Ctx *c, int dtype) {
 }
 int run_chunk(Ctx *c, int dtype, int mode, int batch, const void *field, long long fs, const void *u, long long us,
               const void *w, long long ws, void *ou, long long ous, void *od, long long ods, double *energy,
-              unsigned flags, hipStream_t stream, int epc, int block) {
+              unsigned flags, hipStream_t stream, int epc, int block, const void *wscale) {
   ChunkConfig cfg = default_config(c, dtype);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -423,12 +425,14 @@ int run_chunk(Ctx *c, int dtype, int mode, int batch, const void *field, long lo
   if (block > 0) cfg.block = block;
   if (epc > 0) {
     cfg.epc = epc;
-    return run_chunk_cfg(c, dtype, mode, batch, field, fs, u, us, w, ws, ou, ous, od, ods, energy, flags, stream, cfg);
+    return run_chunk_cfg(c, dtype, mode, batch, field, fs, u, us, w, ws, ou, ous, od, ods, energy, flags, stream, cfg,
+                         nullptr, 0, wscale);
   }
   // a chunk that does not fit LDS (or the 16-bit incidence range) is retried with half the size;
   // the size that worked is remembered for this call shape
   for (bool halved = false;;) {
-    int rc = run_chunk_cfg(c, dtype, mode, batch, field, fs, u, us, w, ws, ou, ous, od, ods, energy, flags, stream, cfg);
+    int rc = run_chunk_cfg(c, dtype, mode, batch, field, fs, u, us, w, ws, ou, ous, od, ods, energy, flags, stream, cfg,
+                           nullptr, 0, wscale);
     if (rc == FEMHOT_OK && halved) {
       std::lock_guard<std::mutex> lk(g_tune_mu);
       g_tuned[{c, mode, dtype, batch, (int)(flags & FEMHOT_ELEMENT_FIELD)}] = cfg;

@@ -22,6 +22,7 @@ struct ChunkArgs {
   long long us;
   const void *w;
   long long ws;
+  const void *wscale;  // optional: a scalar (arithmetic type, device) that multiplies w
   void *ou;
   long long ous;
   void *od;
@@ -147,6 +148,7 @@ __global__ __launch_bounds__(BLOCK, (chunk_min_waves<R, ET, PH, BLOCK>())) void 
   // apart, on 4 of 32 banks; QUAD4 and HEX8 measured no gain from the spare rows)
   const int pad = ET == TET4 ? A.pad : 0;
   R *ERD = ER + (long)(emax * N + cap4 * pad) * P;
+  const R wsc = MODE == MODE_VJP && A.wscale ? *reinterpret_cast<const R *>(A.wscale) : R(1);
   const int tid = threadIdx.x;
   const int n_items = A.n_chunks * A.n_sblocks;
   using UN = typename std::conditional<N == 4, uint2, uint4>::type;  // one element's N uint16
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(BLOCK, (chunk_min_waves<R, ET, PH, BLOCK>())) void 
 #pragma unroll
           for (int c = 0; c < P; ++c) {
             uv[k][c] = Ub[(long long)g[k] * P + c];
-            if constexpr (MODE == MODE_VJP) wv[k][c] = Wb[(long long)g[k] * P + c];
+            if constexpr (MODE == MODE_VJP) wv[k][c] = wsc * Wb[(long long)g[k] * P + c];
           }
           fv[k] = elemental ? R(0) : Fb[g[k]];
         }

@@ -806,7 +806,9 @@ int femhot_ctx_create(const femhot_mesh_desc *d, femhot_ctx **out) {
   // device copies
   std::vector<float> c32(c.h_coords.begin(), c.h_coords.end());
   std::vector<uint8_t> dmask(c.Ndof, 0);
+  std::vector<double> dval(c.Ndof, 0.0);
   for (long long v : c.h_dir_idx) dmask[v] = 1;
+  for (size_t k = 0; k < c.h_dir_idx.size(); ++k) dval[(size_t)c.h_dir_idx[k]] = c.h_dir_val[k];
   auto fail = [&](hipError_t e, const char *what) {
     set_error(std::string("femhot_ctx_create: ") + what + " -> " + hipGetErrorString(e));
     femhot_ctx_destroy(h);
@@ -817,6 +819,7 @@ int femhot_ctx_create(const femhot_mesh_desc *d, femhot_ctx **out) {
   if ((e = hipMalloc(&c.d_coords32, sizeof(float) * c.Nn * 3)) != hipSuccess) return fail(e, "hipMalloc");
   if ((e = hipMalloc(&c.d_conn, sizeof(int) * c.Ne * c.n)) != hipSuccess) return fail(e, "hipMalloc");
   if ((e = hipMalloc(&c.d_dmask, c.Ndof)) != hipSuccess) return fail(e, "hipMalloc");
+  if ((e = hipMalloc(&c.d_dval64, sizeof(double) * c.Ndof)) != hipSuccess) return fail(e, "hipMalloc");
   if ((e = hipMalloc(&c.d_seg_off, sizeof(long long) * (c.nseg + 1))) != hipSuccess) return fail(e, "hipMalloc");
   if ((e = hipMemcpy(c.d_coords64, c.h_coords.data(), sizeof(double) * c.Nn * 3, hipMemcpyHostToDevice)) != hipSuccess)
     return fail(e, "hipMemcpy");
@@ -825,6 +828,8 @@ int femhot_ctx_create(const femhot_mesh_desc *d, femhot_ctx **out) {
   if ((e = hipMemcpy(c.d_conn, c.h_conn.data(), sizeof(int) * c.Ne * c.n, hipMemcpyHostToDevice)) != hipSuccess)
     return fail(e, "hipMemcpy");
   if ((e = hipMemcpy(c.d_dmask, dmask.data(), c.Ndof, hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
+  if ((e = hipMemcpy(c.d_dval64, dval.data(), sizeof(double) * c.Ndof, hipMemcpyHostToDevice)) != hipSuccess)
+    return fail(e, "hipMemcpy");
   if ((e = hipMemcpy(c.d_seg_off, c.h_seg_off.data(), sizeof(long long) * (c.nseg + 1), hipMemcpyHostToDevice)) !=
       hipSuccess)
     return fail(e, "hipMemcpy");
@@ -847,6 +852,7 @@ void femhot_ctx_destroy(femhot_ctx *h) {
   (void)hipFree(c.d_conn);
   (void)hipFree(c.d_dmask);
   (void)hipFree(c.d_seg_off);
+  (void)hipFree(c.d_dval64);
   (void)hipFree(c.d_row_ptr);
   (void)hipFree(c.d_col_idx);
   (void)hipFree(c.d_slot);

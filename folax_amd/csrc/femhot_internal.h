@@ -96,6 +96,7 @@ struct Ctx {
   float *d_coords32 = nullptr;   // (Nn*3)
   int *d_conn = nullptr;         // (Ne*n)
   uint8_t *d_dmask = nullptr;    // (Ndof) 1 = Dirichlet
+  double *d_dval64 = nullptr;    // (Ndof) Dirichlet values (the last entry of a repeated dof), else 0
   long long *d_seg_off = nullptr;  // (nseg+1)
   // lazily built caches
   bool have_pattern = false;

@@ -22,6 +22,7 @@ struct KArgs {
   long long ustride;
   const void *w;
   long long wstride;
+  const void *wscale;  // optional: a scalar (arithmetic type, device) that multiplies w
   void *out_u;  // residual or g_u
   long long oustride;
   void *out_d;  // g_field
@@ -181,11 +182,12 @@ __global__ __launch_bounds__(256) void k_elem(KArgs A) {
       }
     } else if constexpr (MODE == MODE_VJP) {
       const R *W = reinterpret_cast<const R *>(A.w) + (long long)b * A.wstride;
+      const R wsc = A.wscale ? *reinterpret_cast<const R *>(A.wscale) : R(1);
       R w[NL];
 #pragma unroll
       for (int a = 0; a < N; ++a)
 #pragma unroll
-        for (int c = 0; c < P; ++c) w[a * P + c] = W[(size_t)nodes[a] * P + c];
+        for (int c = 0; c < P; ++c) w[a * P + c] = wsc * W[(size_t)nodes[a] * P + c];
       R gu[NL], gd[N];
       elem_vjp<R, ET, PH, NGP>(el, w, A.pp, (A.flags & FEMHOT_PICARD) != 0, gu, gd);
       if (OU) {

@@ -137,6 +137,16 @@ class FiniteElementLoss:
             self.ctx.autotune(op, params, dofs, w, flags=self._flags() & ~L.SCATTER_CHUNK)
             self._tuned.add(key)
 
+    def _one_call(self, bp, bd):
+        """Whether a batch loss runs through its one-call entry points: device tensors of one floating type,
+        fixed Dirichlet values."""
+        return (not self.parametric_boundary_learning and isinstance(bp, torch.Tensor) and isinstance(bd, torch.Tensor)
+                and bd.is_cuda and bp.device == bd.device and bp.dtype == bd.dtype
+                and bd.dtype in (torch.float32, torch.float64) and bp.dim() == 2 and bd.dim() == 2)
+
+    def _has_body_force(self):
+        return bool(np.any(np.asarray(self.loss_settings.get("body_foce", [0.0]), dtype=np.float64) != 0.0))
+
     def _flags(self):
         f = L.ELEMENT_FIELD if self.control_location == "element" else 0
         return f | (L.SCATTER_CHUNK if self.scatter == "chunk" else 0)
@@ -201,6 +211,9 @@ class FiniteElementLoss:
         bp = batch_params if isinstance(batch_params, torch.Tensor) else _as_device_tensor(batch_params, dtype=bd.dtype)
         bp = torch.atleast_2d(bp).reshape(bp.shape[0] if bp.dim() > 1 else 1, -1)
         bd = torch.atleast_2d(bd).reshape(bd.shape[0] if bd.dim() > 1 else 1, -1)
+        if self.loss_function_exponent == 1.0 and self._one_call(bp, bd):
+            m, low, high = _BatchLoss.apply(self, bp, bd)
+            return m, (low, high, m)
         full = _FullDofs.apply(self, bp, bd)
         energies = _BatchEnergy.apply(self, torch.atleast_2d(self.GetParametersVectors(bp)), full)
         be = energies ** self.loss_function_exponent
@@ -266,8 +279,97 @@ class FiniteElementLoss:
         bd = batch_dofs if isinstance(batch_dofs, torch.Tensor) else _as_device_tensor(batch_dofs)
         bp = batch_params if isinstance(batch_params, torch.Tensor) else _as_device_tensor(batch_params, dtype=bd.dtype)
         bp2 = torch.atleast_2d(bp)
+        if self._one_call(bp2, bd):
+            return _BatchResidualNorm.apply(self, bp2, bd, picard)
         full = _FullDofs.apply(self, bp2, torch.atleast_2d(bd))
         return _ResidualNormLoss.apply(self, torch.atleast_2d(self.GetParametersVectors(bp2)), full, picard)
+
+
+class _BatchLoss(torch.autograd.Function):
+    """ComputeBatchLoss with exponent 1 in one library call per pass: (mean, min, max) of the samples'
+    energies.  The residual, which the forward kernel forms anyway, is the energies' gradient with
+    respect to the dofs (see _BatchEnergy), so the backward pass scales it; the control gradient, where
+    asked for, takes the kernels of _BatchEnergy."""
+
+    @staticmethod
+    def forward(ctx, loss, params, dofs):
+        ctx.set_materialize_grads(False)
+        params, dofs = params.contiguous(), dofs.contiguous()
+        loss._tune(L.OP_RESIDUAL, params, dofs)
+        need_p, need_u = ctx.needs_input_grad[1:]
+        mean, low, high, en, full, R = loss.ctx.batch_loss(params, dofs, want_R=need_u, flags=loss._flags())
+        ctx.loss = loss
+        ctx.body = need_u and loss.physics == L.NEOHOOKE and loss._has_body_force()
+        keep_p = ctx.body or (need_p and loss.physics != L.MECHANICAL)
+        ctx.save_for_backward(params if keep_p else None, full if keep_p else None, R, en, low, high)
+        ctx.shape, ctx.dtype = params.shape, dofs.dtype
+        return mean, low, high
+
+    @staticmethod
+    def backward(ctx, g, g_low, g_high):
+        loss = ctx.loss
+        params, full, R, en, low, high = ctx.saved_tensors
+        flags, batch = loss._flags(), en.shape[0]
+        plain = g_low is None and g_high is None and not torch.is_grad_enabled()
+        if plain and g is not None:
+            g = g.contiguous()
+        if not plain:  # each sample's weight: 1 / B of the mean's gradient, the extremes' shared by their ties
+            e = en.sum(dim=1).to(ctx.dtype)
+            s = torch.zeros_like(e) if g is None else (g / batch).expand(batch)
+            for ge, at in ((g_low, low), (g_high, high)):
+                if ge is not None:
+                    tie = (e == at).to(e.dtype)
+                    s = s + ge * tie / tie.sum()
+            s = s.reshape(-1, 1)
+        elif g is None:
+            return None, None, None
+
+        def scaled(t):
+            return loss.ctx.scale(t, g, 1.0 / batch) if plain else t * s
+
+        gu = gd = None
+        if ctx.needs_input_grad[2]:
+            if ctx.body:  # Ee excludes the body-force work: add Fe = -r(u = 0) back
+                r0, _ = loss.ctx.residual(params, torch.zeros_like(full), want_energy=False,
+                                          flags=flags | L.MASK_DIRICHLET)
+                R = R - r0
+            gu = scaled(R)
+        if ctx.needs_input_grad[1]:
+            if loss.physics == L.NEOHOOKE:
+                loss._tune(L.OP_ENERGY_GRAD, params, full)
+                _, _, gd = loss.ctx.energy_grad(params, full, want_gu=False, want_energy=False, flags=flags)
+            elif loss.physics == L.THERMAL:
+                _, gd = loss.ctx.residual_vjp(params, full, full, want_gu=False, flags=flags)
+            gd = scaled(gd) if gd is not None else torch.zeros(ctx.shape, dtype=ctx.dtype, device=en.device)
+        return None, gd, gu
+
+
+class _BatchResidualNorm(torch.autograd.Function):
+    """ComputeBatchResidualNormLoss in one library call per pass; the gradient's incoming factor scales
+    the cotangent inside the VJP kernel, and Dirichlet dofs get none (they are overwritten)."""
+
+    @staticmethod
+    def forward(ctx, loss, params, dofs, picard):
+        params, dofs = params.contiguous(), dofs.contiguous()
+        loss._tune(L.OP_RESIDUAL, params, dofs)
+        value, full, R = loss.ctx.batch_residual_norm(params, dofs, flags=loss._flags())
+        ctx.loss, ctx.picard = loss, picard
+        ctx.save_for_backward(params, full, R)
+        return value
+
+    @staticmethod
+    def backward(ctx, g):
+        loss = ctx.loss
+        params, full, R = ctx.saved_tensors
+        flags = loss._flags() | L.MASK_DIRICHLET | (L.PICARD if ctx.picard else 0)
+        loss._tune(L.OP_VJP, params, full, R)
+        need_p, need_u = ctx.needs_input_grad[1:3]
+        if torch.is_grad_enabled():  # create_graph: the factor stays in the graph
+            gu, gd = loss.ctx.residual_vjp(params, full, R, want_gu=need_u, want_gd=need_p, flags=flags)
+            return None, gd * g if need_p else None, gu * g if need_u else None, None
+        gu, gd = loss.ctx.residual_vjp(params, full, R, want_gu=need_u, want_gd=need_p, flags=flags,
+                                       scale=g.contiguous())
+        return None, gd, gu, None
 
 
 class _FullDofs(torch.autograd.Function):
@@ -319,7 +421,7 @@ class _BatchEnergy(torch.autograd.Function):
         if loss.physics == L.NEOHOOKE:
             loss._tune(L.OP_ENERGY_GRAD, params, dofs)
             _, gu, gd = loss.ctx.energy_grad(params, dofs, want_energy=False, flags=flags)
-            if np.any(np.asarray(loss.loss_settings.get("body_foce", [0.0]), dtype=np.float64) != 0.0):
+            if loss._has_body_force():
                 # Ee excludes the body-force work: add Fe = -r(u = 0) back
                 r0, _ = loss.ctx.residual(params, torch.zeros_like(dofs), want_energy=False, flags=flags)
                 gu = gu - r0

@@ -139,6 +139,33 @@ int femhot_residual_vjp(femhot_ctx *ctx, int dtype, int batch, const void *field
                         long long g_u_stride, void *g_field, long long g_field_stride, unsigned flags,
                         void *stream);
 
+/* femhot_residual_vjp with the cotangent scale * w: scale is a DEVICE scalar of the arithmetic type (NULL:
+ * 1), read by the kernel.  No counterpart in the reference; the backward pass of a scalar loss, whose
+ * incoming gradient is a device scalar. */
+int femhot_residual_vjp_scaled(femhot_ctx *ctx, int dtype, int batch, const void *field, long long field_stride,
+                               const void *u, long long u_stride, const void *w, long long w_stride,
+                               const void *scale, void *g_u, long long g_u_stride, void *g_field,
+                               long long g_field_stride, unsigned flags, void *stream);
+
+/* Residual-norm loss of a batch in one call: full = u with the Dirichlet dofs at their values
+ * (fe_loss.py:91-100), R = the Dirichlet-masked residual of full, loss = 1/2 sum R^2 (FP64 sums).  full, R:
+ * (batch, n_dofs) contiguous; loss: one value of the arithmetic type; scratch: 256 doubles.  flags as for
+ * femhot_residual. */
+int femhot_batch_residual_norm(femhot_ctx *ctx, int dtype, int batch, const void *field, long long field_stride,
+                               const void *u, long long u_stride, void *full, void *R, void *loss, double *scratch,
+                               unsigned flags, void *stream);
+
+/* ComputeBatchLoss (fe_loss.py:250-262, exponent 1) in one call: full as above, energy (batch *
+ * max(1, n_segments)) doubles, mean / low / high over the samples (one value of the arithmetic type each),
+ * and, unless NULL, R = the Dirichlet-masked residual (batch, n_dofs): the gradient of a sample's
+ * energy where the reference takes it so (linear losses; Neo-Hookean without body force). */
+int femhot_batch_loss(femhot_ctx *ctx, int dtype, int batch, const void *field, long long field_stride, const void *u,
+                      long long u_stride, void *full, void *R, double *energy, void *mean, void *low, void *high,
+                      unsigned flags, void *stream);
+
+/* dst[i] = src[i] * (factor * g[0]), i < n, in the arithmetic type; g a DEVICE scalar. */
+int femhot_scale(int dtype, long long n, const void *src, const void *g, double factor, void *dst, void *stream);
+
 /* VJP of the residual with respect to the node coordinates (shape sensitivity): g_x = (dR/dX)^T w,
  * (n_nodes, 3) in the arithmetic type, overwritten; the z column is zero for 2-D elements.  Replaces
  * jax.jacrev(ComputeElement[1], argnums=0) contracted with the element adjoint and assembled per
