@@ -241,8 +241,9 @@ class FemhotContext:
                                              _ptr(gu), self.n_dofs, _ptr(gd), fsz, flags, _stream()))
         return (en.view(B, self.n_segments) if en is not None else None), gu, gd
 
-    def residual_shape_vjp(self, field, u, w, flags=0):
-        """(dR/dX)^T w as an (n_nodes, 3) tensor (one sample): the shape sensitivity of the residual."""
+    def residual_shape_vjp(self, field, u, w, flags=0, wphi=None):
+        """(dR/dX)^T w as an (n_nodes, 3) tensor (one sample): the shape sensitivity of the residual.  wphi
+        (n_elems, G): weights x detJ x integrand of a response whose shape derivative is added."""
         u, w = u.reshape(-1), w.reshape(-1)
         field = field.reshape(-1)
         dt, dev = u.dtype, u.device
@@ -250,9 +251,48 @@ class FemhotContext:
         self._check_in(w.view(1, -1), "w", self.n_dofs, 1, dt, dev)
         self._check_in(field.view(1, -1), "field", self._field_size(flags), 1, dt, dev)
         gx = torch.empty(self.n_nodes, 3, dtype=dt, device=dev)
-        L.check(self._lib.femhot_residual_shape_vjp(self._h, _dtype_code(u), _ptr(field), _ptr(u), _ptr(w), _ptr(gx),
-                                                   flags, _stream()))
+        dim = 2 if self.et == L.QUAD4 else 3
+        if wphi is not None and (wphi.dtype != dt or wphi.device != dev or not wphi.is_contiguous()
+                                 or wphi.numel() % self.n_elems):
+            raise ValueError("wphi must be a contiguous (n_elems, G) tensor of u's dtype and device")
+        scratch = torch.empty(self.n_elems * self.nodes_per_elem * dim, dtype=dt, device=dev)
+        L.check(self._lib.femhot_shape_gradient(self._h, _dtype_code(u), _ptr(field), _ptr(u), _ptr(w), _ptr(wphi),
+                                                _ptr(scratch), _ptr(gx), flags, _stream()))
         return gx
+
+    def build_incidence(self):
+        """The node incidence that gauss_point_gather walks (built by its first call otherwise, not in a
+        capture)."""
+        L.check(self._lib.femhot_incidence(self._h))
+
+    def gauss_point_values(self, field, u, num_gp):
+        """N.d (n_elems, G) and N.u (dofs_per_node, n_elems, G) of a nodal field and a solution."""
+        G = L.gauss_points_per_element(self.et, num_gp)
+        gd = torch.empty(self.n_elems, G, dtype=u.dtype, device=u.device)
+        gu = torch.empty(self.dofs_per_node, self.n_elems, G, dtype=u.dtype, device=u.device)
+        self._check_in(u.view(1, -1), "u", self.n_dofs, 1, u.dtype, u.device)
+        if field.dtype != u.dtype or field.device != u.device or field.numel() < self.n_nodes:
+            raise IndexError(f"field must hold {self.n_nodes} nodal values of u's dtype and device")
+        L.check(self._lib.femhot_gauss_point_values(self._h, _dtype_code(u), _ptr(field), _ptr(u), _ptr(gd), _ptr(gu),
+                                                    _stream()))
+        return gd, gu
+
+    def gauss_point_gather(self, q, num_gp, out=None):
+        """sum over elements and Gauss points of N_a q at the nodes: q (ncomp, n_elems, G) -> (n_nodes, ncomp);
+        out: a contiguous tensor of that shape to add into."""
+        G = L.gauss_points_per_element(self.et, num_gp)
+        q = q.contiguous()
+        if q.dim() != 3 or tuple(q.shape[1:]) != (self.n_elems, G):
+            raise ValueError(f"q must have shape (ncomp, {self.n_elems}, {G})")
+        flags = 0 if out is None else L.ACCUMULATE
+        if out is None:
+            out = torch.empty(self.n_nodes, q.shape[0], dtype=q.dtype, device=q.device)
+        elif out.dtype != q.dtype or out.device != q.device or out.numel() != self.n_nodes * q.shape[0] \
+                or not out.is_contiguous():
+            raise ValueError("out must be a contiguous (n_nodes, ncomp) tensor of q's dtype and device")
+        L.check(self._lib.femhot_gauss_point_gather(self._h, _dtype_code(q), q.shape[0], _ptr(q), _ptr(out), flags,
+                                                    _stream()))
+        return out
 
     def gauss_point_data(self, num_gp, dtype=torch.float64, device=None):
         """Integration data at the context's Gauss rule: N (G, n), w detJ (n_elems, G) and the global

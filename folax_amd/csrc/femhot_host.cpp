@@ -24,6 +24,29 @@ const std::string &get_error() { return g_err; }
 
 static int default_num_gp(int et) { return et == TET4 ? 1 : 2; }
 
+// Node -> (element, local index) incidence, in element order: the row-owner tangent assembly and the
+// gathers of per-corner results walk it.
+int ensure_incidence(Ctx *c) {
+  if (c->d_ne_off) return FEMHOT_OK;
+  const int n = c->n;
+  if (c->Ne * n > 2147483647LL) {
+    set_error("ensure_incidence: more than 2^31 - 1 element corners");
+    return FEMHOT_ERR_SHAPE;
+  }
+  std::vector<int> off(c->Nn + 1, 0), list((size_t)c->Ne * n);
+  for (int g : c->h_conn) off[g + 1]++;
+  for (long long i = 0; i < c->Nn; ++i) off[i + 1] += off[i];
+  std::vector<int> pos(off.begin(), off.end() - 1);
+  for (size_t k = 0; k < list.size(); ++k) list[pos[c->h_conn[k]]++] = (int)k;
+  int *d_off = nullptr;
+  FH_HIP(hipMalloc(&c->d_ne_list, sizeof(int) * list.size()));
+  FH_HIP(hipMemcpy(c->d_ne_list, list.data(), sizeof(int) * list.size(), hipMemcpyHostToDevice));
+  FH_HIP(hipMalloc(&d_off, sizeof(int) * off.size()));
+  FH_HIP(hipMemcpy(d_off, off.data(), sizeof(int) * off.size(), hipMemcpyHostToDevice));
+  c->d_ne_off = d_off;
+  return FEMHOT_OK;
+}
+
 // Build node adjacency (sorted unique neighbour lists incl. self) and the CSR pattern + slot table.
 int ensure_pattern(Ctx *c) {
   if (c->have_pattern) return FEMHOT_OK;
@@ -38,17 +61,10 @@ int ensure_pattern(Ctx *c) {
     for (int a = 0; a < n; ++a) cnt[c->h_conn[e * n + a] + 1]++;
   for (long long i = 0; i < Nn; ++i) cnt[i + 1] += cnt[i];
   std::vector<long long> n2e(cnt[Nn]);
-  // node -> (element, local index) incidence of the row-owner tangent assembly, element order
-  std::vector<int> ne_list(cnt[Nn]), ne_off(Nn + 1);
   {
     std::vector<long long> pos(cnt.begin(), cnt.end() - 1);
     for (long long e = 0; e < Ne; ++e)
-      for (int a = 0; a < n; ++a) {
-        const long long k = pos[c->h_conn[e * n + a]]++;
-        n2e[k] = e;
-        ne_list[k] = (int)(e * n + a);
-      }
-    for (long long i = 0; i <= Nn; ++i) ne_off[i] = (int)cnt[i];
+      for (int a = 0; a < n; ++a) n2e[pos[c->h_conn[e * n + a]]++] = e;
   }
   std::vector<long long> adj_off(Nn + 1, 0);
   std::vector<int> adj;
@@ -123,11 +139,7 @@ int ensure_pattern(Ctx *c) {
   FH_HIP(hipMemcpy(c->d_slot, slot.data(), slot.size(), hipMemcpyHostToDevice));
   FH_HIP(hipMalloc(&c->d_diag_off, sizeof(int) * std::max<long long>(1, c->Ndof)));
   if (c->Ndof) FH_HIP(hipMemcpy(c->d_diag_off, diag_off.data(), sizeof(int) * c->Ndof, hipMemcpyHostToDevice));
-  FH_HIP(hipMalloc(&c->d_ne_off, sizeof(int) * (Nn + 1)));
-  FH_HIP(hipMalloc(&c->d_ne_list, sizeof(int) * std::max<size_t>(1, ne_list.size())));
-  FH_HIP(hipMemcpy(c->d_ne_off, ne_off.data(), sizeof(int) * (Nn + 1), hipMemcpyHostToDevice));
-  if (!ne_list.empty())
-    FH_HIP(hipMemcpy(c->d_ne_list, ne_list.data(), sizeof(int) * ne_list.size(), hipMemcpyHostToDevice));
+  if (int rc = ensure_incidence(c)) return rc;
   c->have_pattern = true;
   return FEMHOT_OK;
 }

@@ -132,6 +132,7 @@ struct Ctx {
 };
 
 int ensure_pattern(Ctx *c);
+int ensure_incidence(Ctx *c);  // d_ne_off, d_ne_list
 int ensure_colouring(Ctx *c);
 // The chunk plan of `epc` elements per chunk, built (and cached) on first use; refused while `s`
 // is being captured into a graph.

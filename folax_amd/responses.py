@@ -7,6 +7,8 @@ and U[c] = N.u_c at each Gauss point, fe_response.py:61-66, 92-113).
 
 What runs where:
 * the Gauss-point geometry (w detJ, N, dN/dx) comes from the library (femhot_gauss_point_data);
+* the nodal field and state are brought to the Gauss points, and Gauss-point terms back to the nodes,
+  by the library's gather kernels;
 * phi is evaluated on the device with torch on all Gauss points at once, and its derivatives with
   respect to the Gauss-point field and state come from torch autograd of that evaluation (the
   formula is arbitrary Python, as the reference's jax.grad of its eval'd lambda);
@@ -18,6 +20,7 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib as L
 from .loss_functions import FiniteElementLoss, _as_device_tensor
 
 
@@ -32,6 +35,40 @@ class _ArrayNamespace:
         if name in self._alias:
             return self._alias[name]
         return getattr(torch, name)
+
+
+class _PointValues(torch.autograd.Function):
+    """N.d and N.u at the Gauss points; its transpose is the gather of _PointGather, so both differentiate
+    to any order."""
+
+    @staticmethod
+    def forward(ctx, loss, d, u):
+        ctx.loss, ctx.n, ctx.shapes = loss, d.numel(), (d.shape, u.shape)
+        return loss.ctx.gauss_point_values(d.contiguous(), u.contiguous(), loss.num_gp)
+
+    @staticmethod
+    def backward(ctx, gd, gu):
+        d = _PointGather.apply(ctx.loss, gd.unsqueeze(0)).reshape(-1) if ctx.needs_input_grad[1] else None
+        if d is not None and ctx.n != d.numel():
+            d = torch.nn.functional.pad(d, (0, ctx.n - d.numel()))
+        return (None, d.reshape(ctx.shapes[0]) if d is not None else None,
+                _PointGather.apply(ctx.loss, gu).reshape(ctx.shapes[1]) if ctx.needs_input_grad[2] else None)
+
+
+class _PointGather(torch.autograd.Function):
+    """sum of N_a q at the nodes, (n_nodes, ncomp); the transpose of _PointValues per component."""
+
+    @staticmethod
+    def forward(ctx, loss, q):
+        ctx.loss, ctx.ncomp = loss, q.shape[0]
+        return loss.ctx.gauss_point_gather(q, loss.num_gp)
+
+    @staticmethod
+    def backward(ctx, g):
+        loss = ctx.loss
+        zero = torch.zeros(loss.ctx.n_dofs, dtype=g.dtype, device=g.device)
+        parts = [_PointValues.apply(loss, g[:, c].contiguous(), zero)[0] for c in range(ctx.ncomp)]
+        return None, torch.stack(parts)
 
 
 class FiniteElementResponse:
@@ -57,7 +94,8 @@ class FiniteElementResponse:
         self.response_function = eval(f"lambda {', '.join(variables)}: {self.response_formula}",
                                       {"jnp": _ArrayNamespace()})
         self._gp = {}
-        self._conn = None
+        self._has_both = False
+        self.fe_loss.ctx.build_incidence()
         self.initialized = True
 
     # ---- Gauss-point integrand ----
@@ -65,9 +103,6 @@ class FiniteElementResponse:
         key = (dtype, device)
         if key not in self._gp:
             self._gp[key] = self.fe_loss.ctx.gauss_point_data(self.fe_loss.num_gp, dtype=dtype, device=device)
-        if self._conn is None or self._conn.device != device:
-            self._conn = torch.as_tensor(self.fe_loss.fe_mesh.GetElementsNodes(self.fe_loss.element_type),
-                                         dtype=torch.int64, device=device)
         return self._gp[key]
 
     def _inputs(self, control, dofs):
@@ -75,53 +110,40 @@ class FiniteElementResponse:
         d = _as_device_tensor(control, dtype=u.dtype, device=u.device)
         return d.reshape(-1), u.reshape(-1)
 
-    def _element_values(self, de, ue, N, wdet):
-        """w detJ phi per element and Gauss point: de (Ne, n), ue (Ne, n, ndpn)."""
-        gp_d = de @ N.T                                  # (Ne, G)
-        gp_u = torch.einsum("ga,eac->ceg", N, ue)        # (ndpn, Ne, G): U[c] is component c
-        return wdet * self.response_function(gp_d, gp_u)
-
-    def _gather(self, d, u):
-        conn = self._conn
-        ndpn = self.fe_loss.number_dofs_per_node
-        return d[conn], u.view(-1, ndpn)[conn]
-
-    def _scatter_nodal(self, vals, width):
-        """Assembles per-element nodal values (Ne, n, width) into (Nn * width,) (fe_response.py:271-272)."""
-        conn = self._conn
-        out = torch.zeros(self.fe_loss.fe_mesh.GetNumberOfNodes(), width, dtype=vals.dtype, device=vals.device)
-        out.index_add_(0, conn.reshape(-1), vals.reshape(-1, width))
-        return out.reshape(-1)
+    def _integrand(self, d, u):
+        """w detJ (Ne, G) and, at the Gauss points, N.d (Ne, G) and N.u (ndpn, Ne, G): U[c] is component c."""
+        _, wdet, _ = self._geometry(u.dtype, u.device)
+        gp_d, gp_u = _PointValues.apply(self.fe_loss, d, u)
+        return wdet, gp_d, gp_u
 
     # ---- reference API ----
     def ComputeValue(self, nodal_control_values, nodal_dof_values):
         """fe_response.py:196-212: sum over elements and Gauss points."""
         d, u = self._inputs(nodal_control_values, nodal_dof_values)
-        N, wdet, _ = self._geometry(u.dtype, u.device)
-        de, ue = self._gather(d, u)
-        return self._element_values(de, ue, N, wdet).sum()
+        wdet, gp_d, gp_u = self._integrand(d, u)
+        return (wdet * self.response_function(gp_d, gp_u)).sum()  # differentiable in both arguments
 
-    def _state_and_control_grads(self, d, u):
-        """d f / d u (Ndof,) and d f / d control (Nn,) of the response integrand alone."""
-        N, wdet, _ = self._geometry(u.dtype, u.device)
-        de, ue = self._gather(d, u)
-        de = de.detach().requires_grad_(True)
-        ue = ue.detach().requires_grad_(True)
+    def _point_grad(self, d, u, which):
+        """Derivative of the response integrand, times w detJ, with respect to the Gauss-point field (which 0:
+        (Ne, G)) or state (1: (ndpn, Ne, G)).  A formula that leaves out either is refused, which the
+        first derivative taken finds out; later ones take the one that is asked for."""
+        wdet, *points = self._integrand(d.detach(), u.detach())
         with torch.enable_grad():
-            f = self._element_values(de, ue, N, wdet).sum()
-            gd, gu = torch.autograd.grad(f, (de, ue))
-        ndpn = self.fe_loss.number_dofs_per_node
-        return self._scatter_nodal(gu, ndpn), self._scatter_nodal(gd.unsqueeze(-1), 1)
+            for k, p in enumerate(points):
+                p.requires_grad_(k == which or not self._has_both)
+            f = self.response_function(*points) * wdet
+            grads = torch.autograd.grad(f, [p for p in points if p.requires_grad], torch.ones_like(f))
+        self._has_both = True
+        return grads[which if len(grads) == 2 else 0]
 
     def ComputeAdjointJacobianMatrixAndRHSVector(self, nodal_control_values, nodal_dof_values):
         """fe_response.py:244-283: rhs = -(df/du) with Dirichlet entries zeroed, and the BC-applied
         transposed tangent of the loss."""
         d, u = self._inputs(nodal_control_values, nodal_dof_values)
-        dfdu, _ = self._state_and_control_grads(d, u)
+        q_u = self._point_grad(d, u, 1)
         idx, _ = self.fe_loss._dir_idx(u.device)
-        rhs = dfdu.clone()
+        rhs = -self.fe_loss.ctx.gauss_point_gather(q_u, self.fe_loss.num_gp).reshape(-1)
         rhs[idx] = 0.0
-        rhs = -rhs
         K, _ = self.fe_loss.ComputeJacobianMatrixAndResidualVector(d, u, transpose_jacobian=True)
         return K, rhs
 
@@ -129,9 +151,12 @@ class FiniteElementResponse:
         """fe_response.py:486-526: df/dk + lambda^T dR/dk (the residual VJP kernel)."""
         d, u = self._inputs(nodal_control_values, nodal_dof_values)
         lam = _as_device_tensor(nodal_adj_dof_values, dtype=u.dtype, device=u.device).reshape(-1)
-        _, dfdk = self._state_and_control_grads(d, u)
-        _, gk = self.fe_loss.ComputeResidualVJP(d, u, lam)
-        return dfdk + gk
+        q_d = self._point_grad(d, u, 0)
+        _, gk = self.fe_loss.ctx.residual_vjp(d.reshape(1, -1), u.reshape(1, -1), lam.reshape(1, -1), want_gu=False,
+                                              flags=self.fe_loss._flags())
+        if gk.numel() != self.fe_loss.ctx.n_nodes:  # an element field: the two have no common length
+            return self.fe_loss.ctx.gauss_point_gather(q_d.unsqueeze(0), self.fe_loss.num_gp).reshape(-1) + gk[0]
+        return self.fe_loss.ctx.gauss_point_gather(q_d.unsqueeze(0), self.fe_loss.num_gp, out=gk).reshape(-1)
 
     def ComputeAdjointNodalShapeDerivatives(self, nodal_control_values, nodal_dof_values, nodal_adj_dof_values):
         """fe_response.py:365-406: df/dX + lambda^T dR/dX, flattened (3 n_nodes,).  Only detJ of the
@@ -139,14 +164,22 @@ class FiniteElementResponse:
         residual term runs in the shape-VJP kernel."""
         d, u = self._inputs(nodal_control_values, nodal_dof_values)
         lam = _as_device_tensor(nodal_adj_dof_values, dtype=u.dtype, device=u.device).reshape(-1)
-        N, wdet, dndx = self._geometry(u.dtype, u.device)
-        de, ue = self._gather(d, u)
-        wphi = self._element_values(de, ue, N, wdet)                  # (Ne, G)
-        ge = torch.einsum("eg,egaj->eaj", wphi, dndx)                # (Ne, n, dim)
-        if ge.shape[-1] < 3:
-            ge = torch.nn.functional.pad(ge, (0, 3 - ge.shape[-1]))
-        dfdX = self._scatter_nodal(ge, 3)
-        return dfdX + self.fe_loss.ComputeResidualShapeVJP(d, u, lam)
+        wdet, gp_d, gp_u = self._integrand(d, u)
+        wphi = (wdet * self.response_function(gp_d, gp_u)).contiguous()
+        if wphi.shape != wdet.shape:
+            raise RuntimeError(f"the response formula must give one value per Gauss point, got {tuple(wphi.shape)}")
+        if wphi.requires_grad:  # the caller differentiates the integrand's part
+            _, _, dndx = self._geometry(u.dtype, u.device)
+            ge = torch.einsum("eg,egaj->eaj", wphi, dndx)                # (Ne, n, dim)
+            if ge.shape[-1] < 3:
+                ge = torch.nn.functional.pad(ge, (0, 3 - ge.shape[-1]))
+            conn = torch.as_tensor(self.fe_loss.fe_mesh.GetElementsNodes(self.fe_loss.element_type),
+                                   dtype=torch.int64, device=u.device)
+            dfdX = torch.zeros(self.fe_loss.fe_mesh.GetNumberOfNodes(), 3, dtype=u.dtype, device=u.device)
+            dfdX.index_add_(0, conn.reshape(-1), ge.reshape(-1, 3))
+            return dfdX.reshape(-1) + self.fe_loss.ComputeResidualShapeVJP(d, u, lam)
+        flags = L.ELEMENT_FIELD if self.fe_loss.control_location == "element" else 0
+        return self.fe_loss.ctx.residual_shape_vjp(d, u, lam, flags=flags, wphi=wphi).reshape(-1)
 
     def Finalize(self):
         pass

@@ -174,6 +174,23 @@ int femhot_scale(int dtype, long long n, const void *src, const void *g, double 
 int femhot_residual_shape_vjp(femhot_ctx *ctx, int dtype, const void *field, const void *u, const void *w,
                               void *g_x, unsigned flags, void *stream);
 
+/* femhot_residual_shape_vjp plus the shape derivative of an integrand, summed per node in element order:
+ * g_x = (dR/dX)^T w + sum_e sum_g wphi(e, g) dN/dx, with wphi (n_elems, G) = weight x detJ x integrand at the
+ * Gauss points (NULL: none; fe_response.py:365-406).  scratch: n_elems * nodes_per_elem * dim values. */
+int femhot_shape_gradient(femhot_ctx *ctx, int dtype, const void *field, const void *u, const void *w,
+                          const void *wphi, void *scratch, void *g_x, unsigned flags, void *stream);
+
+/* The two sides of a response formula (fe_response.py:92-113, 271-272): a nodal field (n_nodes) and the
+ * solution (n_dofs) at the Gauss points, gp_field (n_elems, G) and gp_u (dofs_per_node, n_elems, G); and
+ * Gauss-point terms back at the nodes, out(node, c) = sum_(e, a at node) sum_g N_a(g) q(c, e, g) for q (ncomp,
+ * n_elems, G), out (n_nodes, ncomp), overwritten unless FEMHOT_ACCUMULATE.  The gather walks the context's
+ * node incidence, built by its first call or, for callers that capture it, by femhot_incidence. */
+int femhot_incidence(femhot_ctx *ctx);
+int femhot_gauss_point_values(femhot_ctx *ctx, int dtype, const void *field, const void *u, void *gp_field,
+                              void *gp_u, void *stream);
+int femhot_gauss_point_gather(femhot_ctx *ctx, int dtype, int ncomp, const void *q, void *out, unsigned flags,
+                              void *stream);
+
 /* femhot_energy_grad that allocates nothing: no counterpart in the reference; for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same arguments and results as femhot_energy_grad on the LDS-staged chunk path (the
