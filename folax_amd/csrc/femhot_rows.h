@@ -10,8 +10,9 @@
 //   2. lane (element s, node b) forms block (a, b) of the element tangent (a = local index of i in
 //      s), Dirichlet-masked, stores it in LDS and sets its bit in the mask of its column k (the
 //      position of node b among i's neighbours, from the slot table);
-//   3. lane per output value (row c, column k, component d) adds the blocks of the lanes in column
-//      k's mask, in lane order (element order, then b), to its register accumulator.
+//   3. lane per output value (row c, column k, component d; CPW columns per round, so a lane keeps its row
+//      and component) adds the blocks of the lanes in column k's mask, in lane order (element order,
+//      then b), to its register accumulator.
 // Columns are taken KW at a time; one window covers every node of hexahedral and tetrahedral meshes
 // of ordinary valence, and a wider node repeats the batches once per window.
 //
@@ -61,16 +62,16 @@ __device__ __forceinline__ R gp_inverse(int g, const double *xs, R (&Nv)[ElemT<E
   constexpr int N = ElemT<ET>::N, D = ElemT<ET>::D;
   double xi, eta, zeta, w;
   gauss_point<ET, NGP>(g, xi, eta, zeta, w);
-  if constexpr (ET == HEX8) {
+  if constexpr (ET == HEX8) {  // xs holds the coordinates' moments (hex8_lane_moment)
     R J[3][3];  // 8 J
     const R X = R(xi), Y = R(eta), Z = R(zeta), XY = R(xi * eta), XZ = R(xi * zeta), YZ = R(eta * zeta);
+    constexpr int lane_of[8] = {0, 1, 3, 4, 2, 5, 7, 6};  // the lane that holds moment m
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      R col[8], m[8];
-      col[0] = R(0);
+      R m[8];
+      m[0] = R(0);
 #pragma unroll
-      for (int a = 1; a < 8; ++a) col[a] = R(xs[a * 3 + i] - xs[i]);
-      hex8_moments<R>(col, m);
+      for (int k = 1; k < 8; ++k) m[k] = R(xs[lane_of[k] * 3 + i]);
       hex8_dxi<R>(m, X, Y, Z, XY, XZ, YZ, J[i]);
     }
 #pragma unroll
@@ -190,11 +191,36 @@ __device__ __forceinline__ void stage_gradients(int g, const R (&inv)[ElemT<ET>:
   }
 }
 
+// Coordinate of a HEX8 node -> moment of the element's coordinates (hex8_moments' sums, in its order), across
+// the 8 lanes that hold the element's nodes 0..7: coordinates relative to node 0, then one butterfly per
+// reference direction with DPP register moves.  Lane b ends with the moment whose sign product is that of
+// the directions in which node b lies on the + side: moment lane_of^-1 of gp_inverse.  Formed
+// once per element where every Gauss-point lane formed all of them (93 FP64 adds each).
+template <int CTRL, int BANKS> __device__ __forceinline__ double rows_dpp_into(double old, double v) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, 0xf, BANKS, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf, BANKS, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double hex8_lane_moment(double v, int b) {
+  // node 0's value: lane 0 of the lower and lane 8 of the upper half of each row of 16 (row_newbcast)
+  double ref = rows_dpp_into<0x150, 0x3>(v, v);
+  ref = rows_dpp_into<0x158, 0xc>(ref, v);
+  v -= ref;
+  const double sx = (b & 3) == 1 || (b & 3) == 2 ? -1.0 : 1.0, sy = (b & 3) >= 2 ? -1.0 : 1.0, sz = b >= 4 ? -1.0 : 1.0;
+  // the lane on the - side adds its partner, the one on the + side subtracts it (products by +-1 are exact)
+  v = __builtin_fma(sx, rows_dpp_into<0xB1, 0xf>(0.0, v), v);  // b ^ 1 (quad_perm [1,0,3,2])
+  v = __builtin_fma(sy, rows_dpp_into<0x1B, 0xf>(0.0, v), v);  // b ^ 3 (quad_perm [3,2,1,0])
+  double up = rows_dpp_into<0x104, 0x5>(0.0, v);               // b ^ 4: row_shl:4 into banks 0 and 2,
+  up = rows_dpp_into<0x114, 0xa>(up, v);                       // row_shr:4 into banks 1 and 3
+  return __builtin_fma(sz, up, v);
+}
+
 template <int ET, int NGP, int N, int P> struct RowsShape {
   static constexpr int G = RuleSize<ET, NGP>::G;
+  static constexpr int CPW = 64 / (P * P);                         // columns per round of the output stage
   static constexpr int EB = (64 / G < 64 / N) ? 64 / G : 64 / N;  // incident elements per batch
   static constexpr int KW = (P == 3) ? 28 : 64;                    // neighbour columns per window
-  static constexpr int OR = (P * P * KW + 63) / 64;                // output values per lane per window
+  static constexpr int OR = (KW + CPW - 1) / CPW;                  // output values per lane per window
 };
 
 // Waves per SIMD the compiler must fit: 3 for linear elasticity (168 VGPRs in FP64 HEX8 2x2x2, no spills);
@@ -207,7 +233,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
   using E = Elem<R, ET, PH>;
   constexpr int N = E::N, D = E::D, P = E::P;
   using SH = RowsShape<ET, NGP, N, P>;
-  constexpr int G = SH::G, EB = SH::EB, KW = SH::KW, OR = SH::OR;
+  constexpr int G = SH::G, EB = SH::EB, KW = SH::KW, OR = SH::OR, CPW = SH::CPW;
   constexpr int UNR = G <= 8 ? G : 1;
   constexpr int ST = N * D + 1;  // staged values per (element, Gauss point): dN/dx of N nodes, f_g
   constexpr int SW = (EB * G * ST > 64 * P * P) ? EB * G * ST : 64 * P * P;
@@ -217,7 +243,9 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
   // lane's writes depend on its reads, and the workgroup is one wave), so the two never overlap in
   // time and the workgroup needs no extra LDS.
   constexpr int XW = (64 * 3 * 8 + 2 * 64 * (int)sizeof(R)) / (int)sizeof(R);  // a multiple of 4
-  constexpr int SX = ((SW > XW ? SW : XW) + 3) & ~3;  // so XS starts 16-byte aligned
+  // (the output stage reads up to 3 blocks past a column's last: 4 more blocks stay in bounds)
+  constexpr int SB = SW > (64 + 4) * P * P ? SW : (64 + 4) * P * P;
+  constexpr int SX = ((SB > XW ? SB : XW) + 3) & ~3;  // so XS starts 16-byte aligned
   __shared__ __align__(16) R S[SX];
   __shared__ unsigned long long MK[KW];
   __shared__ int CS[KW + 1];
@@ -247,28 +275,11 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
   R *V = reinterpret_cast<R *>(A.vals) + rp;
   const int s2 = lane / N, b2 = lane - s2 * N;  // lane (element, node) of steps 0 and 2
   const int s1 = lane / G, g1 = lane - s1 * G;  // lane (element, Gauss point) of step 1
+  // lane of the output stage: row oc, column kk of a round's CPW, component od (row by row, so a round
+  // writes P runs of CPW * P values); lanes past P rows idle
+  const int oc = lane / (CPW * P), kk = (lane - oc * CPW * P) / P, od = lane - oc * CPW * P - kk * P;
   for (int k0 = 0; k0 < deg; k0 += KW) {
-    const int kw = min(KW, deg - k0), nout = P * P * kw;
-    // this lane's outputs in the window: t = r * 64 + lane -> row c, column k0 + k, component d, at
-    // offset oo in the node's P rows (row c starts at c * P * deg); no integer division by kw
-    int ok[OR], ocd[OR], oo[OR];
-    const int pk = P * kw, pdeg = P * deg;
-#pragma unroll
-    for (int r = 0; r < OR; ++r) {
-      const int t = r * 64 + lane;
-      int c = 0, cs = 0, cr = 0;
-#pragma unroll
-      for (int q = 1; q < P; ++q) {
-        const bool ge = t >= cs + pk;
-        c += ge ? 1 : 0;
-        cs += ge ? pk : 0;
-        cr += ge ? pdeg : 0;
-      }
-      const int rem = t - cs, k = rem / P;
-      ok[r] = t < nout ? k : -1;
-      ocd[r] = c * P + (rem - k * P);
-      oo[r] = cr + k0 * P + rem;
-    }
+    const int kw = min(KW, deg - k0);
     R acc[OR];
 #pragma unroll
     for (int r = 0; r < OR; ++r) acc[r] = R(0);
@@ -277,6 +288,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       // 0. lane (s, b) fetches node b of incident element s: coordinates, field and (thermal)
       //    solution to LDS; its column among the owned node's neighbours stays in a register
       int a2 = 0, col = -1;
+      double xc[3] = {0.0, 0.0, 0.0};
       if (s2 < nb) {
         const int ea = A.ne_list[off0 + base + s2];
         const int e = ea / N;
@@ -284,10 +296,12 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         col = A.slot[((size_t)e * N + a2) * N + b2];
         const int nd = A.conn[(size_t)e * N + b2];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) XS[lane * 3 + i] = A.coords[(size_t)nd * 3 + i];
+        for (int i = 0; i < 3; ++i) xc[i] = A.coords[(size_t)nd * 3 + i];
         FS[lane] = elemental ? F[e] : F[nd];
         if constexpr (PH == THERMAL) US[lane] = U[nd];
       }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) XS[lane * 3 + i] = ET == HEX8 ? hex8_lane_moment(xc[i], b2) : xc[i];
       for (int t = lane; t < kw; t += 64) MK[t] = 0ull;
       __syncthreads();
       // the lanes of each column of the window, as a bit mask
@@ -333,19 +347,19 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       __syncthreads();
       {  // blocks are stored column by column, lanes in order: CS[k] = first block of column k
         int pc = lane < kw ? __popcll(MK[lane]) : 0;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const int y = __shfl_up(pc, o);
-          if (lane >= o) pc += y;
-        }
+        pc += __builtin_amdgcn_update_dpp(0, pc, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8: sums in rows of 16
+        pc += __builtin_amdgcn_update_dpp(0, pc, 0x112, 0xf, 0xf, true);
+        pc += __builtin_amdgcn_update_dpp(0, pc, 0x114, 0xf, 0xf, true);
+        pc += __builtin_amdgcn_update_dpp(0, pc, 0x118, 0xf, 0xf, true);
+        pc += __builtin_amdgcn_update_dpp(0, pc, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+        pc += __builtin_amdgcn_update_dpp(0, pc, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
         if (lane < kw) CS[lane + 1] = pc;
         if (lane == 0) CS[0] = 0;
       }
       R K[P * P];
-#pragma unroll
-      for (int i = 0; i < P * P; ++i) K[i] = R(0);
-      if (s2 < nb) {  // 2. block (a, b) of each incident element's tangent
-        const int a = a2, b = b2;
+      {  // 2. block (a, b) of each incident element's tangent (lanes past the batch's elements form one that
+         // is not stored, from whatever their slots hold)
+        const int a = a2, b = b2, sb = 64 / N > EB ? min(s2, EB - 1) : s2;
         R M[D][D];
 #pragma unroll
         for (int p = 0; p < D; ++p)
@@ -354,7 +368,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         R t = R(-0.0);
 #pragma unroll UNR
         for (int g = 0; g < G; ++g) {
-          const R *st = S + (s2 * G + g) * ST;
+          const R *st = S + (sb * G + g) * ST;
           const R f = st[N * D];
           R fa[D], db[D];
 #pragma unroll
@@ -393,6 +407,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         // a Dirichlet row keeps only the element diagonal (fe_loss.py:191-207); dm is the same for
         // the whole workgroup, so free nodes skip this
         if (any_dm) {
+          asm volatile("" ::: "memory");  // keeps this a branch: the selects would run for every node
 #pragma unroll
           for (int c = 0; c < P; ++c)
 #pragma unroll
@@ -410,13 +425,15 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       __syncthreads();
 #pragma unroll
       for (int r = 0; r < OR; ++r) {  // 3. each output sums its column's blocks in lane order
-        if (ok[r] < 0) continue;
-        const int lo = CS[ok[r]], hi = CS[ok[r] + 1];
+        const int k = r * CPW + kk;
+        if (k >= kw || oc >= P) continue;
+        const int lo = CS[k], hi = CS[k + 1];
         R sum = R(0);
         for (int i = lo; i < hi; i += 4) {  // four contributions per round, their loads issued together
+          const R *src = S + i * (P * P) + oc * P + od;
           R x[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) x[q] = S[min(i + q, hi - 1) * P * P + ocd[r]];
+          for (int q = 0; q < 4; ++q) x[q] = src[q * P * P];
 #pragma unroll
           for (int q = 0; q < 4; ++q) sum += (i + q < hi) ? x[q] : R(0);
         }
@@ -426,8 +443,9 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
     }
 #pragma unroll
     for (int r = 0; r < OR; ++r) {
-      if (ok[r] < 0) continue;
-      R *v = V + oo[r];
+      const int k = r * CPW + kk;
+      if (k >= kw || oc >= P) continue;
+      R *v = V + oc * P * deg + (k0 + k) * P + od;
       *v = accumulate ? *v + acc[r] : acc[r];
     }
   }
