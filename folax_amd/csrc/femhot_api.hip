@@ -276,9 +276,8 @@ int femhot_tangent_csr(femhot_ctx *h, int dtype, const void *field, const void *
     if (path == PATH_COLOUR) flags |= FEMHOT_SCATTER_COLOUR;
     if (path == PATH_ROWS) flags |= FEMHOT_SCATTER_ROWS;
   }
-  // row-owner assembly covers thermal and linear elasticity (and grids of up to 2^26 nodes of 64
-  // lanes); otherwise the call takes colour-ordered adds
-  const bool rows = (flags & FEMHOT_SCATTER_ROWS) && c->ph != NEOHOOKE && c->Nn <= (1LL << 26);
+  // where the row-owner assembly does not cover the context the call takes colour-ordered adds
+  const bool rows = (flags & FEMHOT_SCATTER_ROWS) && rows_tangent(c);
   if ((flags & FEMHOT_SCATTER_ROWS) && !rows) flags |= FEMHOT_SCATTER_COLOUR;
   if (!acc && !rows) {
     rc = dtype == FEMHOT_F32 ? fill<float>((float *)vals, c->nnz, c->nnz, 1, 0.f, s)
@@ -379,7 +378,7 @@ int femhot_autotune(femhot_ctx *h, int op, int dtype, int batch, const void *fie
     const unsigned tf = flags & (FEMHOT_ELEMENT_FIELD | FEMHOT_TRANSPOSE);
     FH_HIP(hipEventCreate(&e0));
     FH_HIP(hipEventCreate(&e1));
-    const bool rows_ok = c->ph != NEOHOOKE && c->Nn <= (1LL << 26);
+    const bool rows_ok = rows_tangent(c);
     float t_atomic = 0.f, t_colour = 0.f, t_rows = 0.f;
     int rc = time_it([&] { return femhot_tangent_csr(h, dtype, field, u, out_u, nullptr, tf, stream); }, &t_atomic);
     if (!rc)

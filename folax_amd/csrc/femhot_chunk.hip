@@ -553,7 +553,7 @@ int tuned_path(const Ctx *c, int dtype, int mode, int batch, unsigned flags) {
     auto it = g_tuned.find({c, mode, dtype, batch, (int)(flags & FEMHOT_ELEMENT_FIELD)});
     if (it != g_tuned.end()) return it->second.path;
   }
-  if (mode == MODE_TANGENT) return c->ph == NEOHOOKE ? PATH_COLOUR : PATH_ROWS;
+  if (mode == MODE_TANGENT) return rows_tangent(c) ? PATH_ROWS : PATH_COLOUR;
   return (dtype == FEMHOT_F64 && c->ph == NEOHOOKE) ? PATH_ATOMIC : PATH_CHUNK;
 }
 

@@ -145,6 +145,12 @@ void free_chunk_plans(Ctx *c);
 int init_fixed_scratch();
 int ensure_workspace(Ctx *c, size_t bytes);
 
+// Whether the row-owner tangent assembly covers the context: thermal and linear elasticity, Neo-Hookean on
+// HEX8 at the 2x2x2 rule; grids of up to 2^26 nodes.
+inline bool rows_tangent(const Ctx *c) {
+  return (c->ph != NEOHOOKE || (c->et == HEX8 && c->ngp == 2)) && c->Nn <= (1LL << 26);
+}
+
 // Records an event on `s` when timing is enabled (pairs: before/after the dominant kernel).
 int timing_mark(Ctx *c, hipStream_t s);
 

@@ -55,6 +55,12 @@ template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_f64(double v
   return __hiloint2double(hi, lo);
 }
 
+// v of the lane that DPP control CTRL names (every lane has one).
+template <int CTRL> __device__ __forceinline__ double lane_dpp(double v) { return dpp_f64<CTRL, 0xf>(v); }
+template <int CTRL> __device__ __forceinline__ float lane_dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
 // Sum over the 64 lanes of a wave, valid in lane 63 only: pairs and quads (quad_perm), half rows and
 // rows (row_half_mirror, row_mirror), then row 0 into row 1 and row 2 into row 3 (row_bcast:15), then
 // rows 0-1 into rows 2-3 (row_bcast:31).  Register moves instead of the LDS round trips of a shuffle

@@ -3,7 +3,7 @@
 #include <type_traits>
 
 #include "femhot_kernels.h"
-#include "femhot_rows.h"
+#include "femhot_rows_hex8.h"
 
 namespace femhot {
 
@@ -75,8 +75,12 @@ template <int ET> int launch_tangent_impl(const TangentLaunch &L) {
     using R = std::remove_pointer_t<decltype(rp)>;
     constexpr int PH = decltype(phc)::value, NGP = decltype(ngpc)::value;
     if (L.rows) {
-      if constexpr (PH == NEOHOOKE) {
-        set_error("femhot_tangent_csr: the row-owner assembly covers thermal and linear-elastic physics");
+      if constexpr (ET == HEX8 && NGP == 2) {
+        hipLaunchKernelGGL((k_tangent_rows_hex8<R, PH>), L.grid, dim3(64), 0, L.stream, L.args);
+        FH_HIP(hipGetLastError());
+        return FEMHOT_OK;
+      } else if constexpr (PH == NEOHOOKE) {
+        set_error("femhot_tangent_csr: the row-owner assembly of Neo-Hookean covers HEX8 at the 2x2x2 rule");
         return FEMHOT_ERR_UNSUPPORTED;
       } else {
         hipLaunchKernelGGL((k_tangent_rows<R, ET, PH, NGP>), L.grid, dim3(64), 0, L.stream, L.args);

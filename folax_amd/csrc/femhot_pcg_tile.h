@@ -91,18 +91,13 @@ template <class T> __device__ __forceinline__ T tile_wait(const T *p, typename T
 // Every store of this wave has reached the memory other workgroups read.
 __device__ __forceinline__ void tile_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// v of the lane that DPP control CTRL names (every lane has one).
-template <int CTRL> __device__ __forceinline__ double tile_dpp(double v) { return dpp_f64<CTRL, 0xf>(v); }
-template <int CTRL> __device__ __forceinline__ float tile_dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
 // Sum over each aligned group of N lanes (4, 8 or 16), held by all of them: quad_perm [1,0,3,2] and
 // [2,3,0,1], then row_half_mirror and row_mirror, which pair lanes of equal sums.
 template <int N, class T> __device__ __forceinline__ T tile_lane_sum(T v) {
-  v += tile_dpp<0xB1>(v);
-  v += tile_dpp<0x4E>(v);
-  if constexpr (N >= 8) v += tile_dpp<0x141>(v);
-  if constexpr (N >= 16) v += tile_dpp<0x140>(v);
+  v += lane_dpp<0xB1>(v);
+  v += lane_dpp<0x4E>(v);
+  if constexpr (N >= 8) v += lane_dpp<0x141>(v);
+  if constexpr (N >= 16) v += lane_dpp<0x140>(v);
   return v;
 }
 

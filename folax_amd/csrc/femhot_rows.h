@@ -223,6 +223,54 @@ template <int ET, int NGP, int N, int P> struct RowsShape {
   static constexpr int OR = (KW + CPW - 1) / CPW;                  // output values per lane per window
 };
 
+// CS[k] = first block of column k: exclusive prefix sums of the columns' lane counts, by DPP register moves.
+template <int KW>
+__device__ __forceinline__ void rows_column_starts(int lane, int kw, const unsigned long long *MK, int *CS) {
+  int pc = lane < kw ? __popcll(MK[lane]) : 0;
+  pc += __builtin_amdgcn_update_dpp(0, pc, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8: sums in rows of 16
+  pc += __builtin_amdgcn_update_dpp(0, pc, 0x112, 0xf, 0xf, true);
+  pc += __builtin_amdgcn_update_dpp(0, pc, 0x114, 0xf, 0xf, true);
+  pc += __builtin_amdgcn_update_dpp(0, pc, 0x118, 0xf, 0xf, true);
+  pc += __builtin_amdgcn_update_dpp(0, pc, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  pc += __builtin_amdgcn_update_dpp(0, pc, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  if (lane < kw) CS[lane + 1] = pc;
+  if (lane == 0) CS[0] = 0;
+}
+
+// Output stage: a lane owns row oc, component od and column kk of each round's CPW, and adds the column's
+// blocks in lane order (S reaches 3 blocks past the last).
+template <class R, int P, int CPW, int OR>
+__device__ __forceinline__ void rows_add_columns(int kw, int oc, int kk, int od, const R *S, const int *CS,
+                                                 R (&acc)[OR]) {
+#pragma unroll
+  for (int r = 0; r < OR; ++r) {
+    const int k = r * CPW + kk;
+    if (k >= kw || oc >= P) continue;
+    const int lo = CS[k], hi = CS[k + 1];
+    R sum = R(0);
+    for (int i = lo; i < hi; i += 4) {  // four contributions per round, their loads issued together
+      const R *src = S + i * (P * P) + oc * P + od;
+      R x[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[q] = src[q * P * P];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sum += (i + q < hi) ? x[q] : R(0);
+    }
+    acc[r] += sum;
+  }
+}
+template <class R, int P, int CPW, int OR>
+__device__ __forceinline__ void rows_write(int kw, int k0, int deg, int oc, int kk, int od, bool accumulate,
+                                           const R (&acc)[OR], R *V) {
+#pragma unroll
+  for (int r = 0; r < OR; ++r) {
+    const int k = r * CPW + kk;
+    if (k >= kw || oc >= P) continue;
+    R *v = V + oc * P * deg + (k0 + k) * P + od;
+    *v = accumulate ? *v + acc[r] : acc[r];
+  }
+}
+
 // Waves per SIMD the compiler must fit: 3 for linear elasticity (168 VGPRs in FP64 HEX8 2x2x2, no spills);
 // the thermal instantiations keep the compiler's own choice (the powc of k(T) would spill under 3).
 template <int PH> constexpr int rows_min_waves() { return PH == MECH ? 3 : 1; }
@@ -346,15 +394,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       }
       __syncthreads();
       {  // blocks are stored column by column, lanes in order: CS[k] = first block of column k
-        int pc = lane < kw ? __popcll(MK[lane]) : 0;
-        pc += __builtin_amdgcn_update_dpp(0, pc, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8: sums in rows of 16
-        pc += __builtin_amdgcn_update_dpp(0, pc, 0x112, 0xf, 0xf, true);
-        pc += __builtin_amdgcn_update_dpp(0, pc, 0x114, 0xf, 0xf, true);
-        pc += __builtin_amdgcn_update_dpp(0, pc, 0x118, 0xf, 0xf, true);
-        pc += __builtin_amdgcn_update_dpp(0, pc, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-        pc += __builtin_amdgcn_update_dpp(0, pc, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
-        if (lane < kw) CS[lane + 1] = pc;
-        if (lane == 0) CS[0] = 0;
+        rows_column_starts<KW>(lane, kw, MK, CS);
       }
       R K[P * P];
       {  // 2. block (a, b) of each incident element's tangent (lanes past the batch's elements form one that
@@ -423,31 +463,10 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         for (int i = 0; i < P * P; ++i) S[dst * P * P + i] = K[i];
       }
       __syncthreads();
-#pragma unroll
-      for (int r = 0; r < OR; ++r) {  // 3. each output sums its column's blocks in lane order
-        const int k = r * CPW + kk;
-        if (k >= kw || oc >= P) continue;
-        const int lo = CS[k], hi = CS[k + 1];
-        R sum = R(0);
-        for (int i = lo; i < hi; i += 4) {  // four contributions per round, their loads issued together
-          const R *src = S + i * (P * P) + oc * P + od;
-          R x[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) x[q] = src[q * P * P];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) sum += (i + q < hi) ? x[q] : R(0);
-        }
-        acc[r] += sum;
-      }
+      rows_add_columns<R, P, CPW, OR>(kw, oc, kk, od, S, CS, acc);  // 3. each output sums its column's blocks
       __syncthreads();  // before the next batch overwrites the blocks and the masks
     }
-#pragma unroll
-    for (int r = 0; r < OR; ++r) {
-      const int k = r * CPW + kk;
-      if (k >= kw || oc >= P) continue;
-      R *v = V + oc * P * deg + (k0 + k) * P + od;
-      *v = accumulate ? *v + acc[r] : acc[r];
-    }
+    rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
   }
 }
 

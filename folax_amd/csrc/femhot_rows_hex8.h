@@ -1,0 +1,236 @@
+// Row-owner tangent assembly for HEX8 at the 2x2x2 rule (see femhot_rows.h for the assembly itself: one
+// 64-lane workgroup per node, its incident elements' blocks summed per column in a fixed order).
+//
+// The 8 lanes of an element are its 8 nodes and its 8 Gauss points at once: with the Gauss coordinates
+// +-s, s = 1/sqrt(3), the trilinear shape functions are products of 2 x 2 matrices, one per reference
+// direction, so every map between nodal and Gauss-point values is three butterflies between the lanes
+// whose node (point) lies across that direction:
+//   B: v + g p   (interpolation; g = (1 - s) / (1 + s), times 1 + s)
+//   D: the difference quotient across the direction (s v - s p from nodes to points, s (v + p) back)
+// with v the lane's own value and p its partner's.  J, the field, the temperature and the displacement
+// gradient come from the nodes by them, and the blocks sum_g f dN_a (x) dN_b of all 8 nodes b go back
+// by the transposed ones.  Nothing is staged in LDS (the general kernel stages 25 values per Gauss
+// point and reads 56 back per lane, which kept its LDS busy for half its time and allowed 3 waves
+// per SIMD), and each of the blocks' 9 entries costs 26 instructions.  A lane's partners are lane ^ 1, ^ 3
+// and ^ 7, one DPP move per 32 bits: lanes 4..7 hold the upper nodes in the order 7, 6, 5, 4.
+//
+// Bound: FP64 vector issue.  MEASURED
+#pragma once
+#include "femhot_rows.h"
+
+namespace femhot {
+
+template <int DIR, class T> __device__ __forceinline__ T hex8_across(T v) {
+  return lane_dpp<DIR == 0 ? 0xB1 : DIR == 1 ? 0x1B : 0x141>(v);  // quad_perm [1,0,3,2], [3,2,1,0], row_half_mirror
+}
+
+constexpr double HEX8_S = 0.57735026918962576451;  // 1/sqrt(3)
+constexpr double HEX8_G = (1.0 - HEX8_S) / (1.0 + HEX8_S);
+
+// Node values -> their derivatives along the reference directions at the lane's point, over (1 + s)^2 / 8.
+// sg: the lane's signs.
+template <class R> __device__ __forceinline__ void hex8_point_gradient(R v, const R (&sg)[3], R (&o)[3]) {
+  const R g = R(HEX8_G);
+  const R px = hex8_across<0>(v), u = sg[0] * (v - px), w = v + g * px;
+  const R yu = u + g * hex8_across<1>(u), pw = hex8_across<1>(w), dw = sg[1] * (w - pw), bw = w + g * pw;
+  o[0] = yu + g * hex8_across<2>(yu);
+  o[1] = dw + g * hex8_across<2>(dw);
+  o[2] = sg[2] * (bw - hex8_across<2>(bw));
+}
+// Node values -> the value at the lane's point, over (1 + s)^3 / 8.
+template <class R> __device__ __forceinline__ R hex8_point_value(R v) {
+  const R g = R(HEX8_G);
+  v += g * hex8_across<0>(v);
+  v += g * hex8_across<1>(v);
+  return v + g * hex8_across<2>(v);
+}
+// sum over the points of sum_k q_k dN_b/dxi_k for the lane's node b, over (1 + s)^2 / 8; q_k carries the
+// lane's sign along k.
+template <class R> __device__ __forceinline__ R hex8_node_sum(R q0, R q1, R q2) {
+  const R g = R(HEX8_G);
+  const R u0 = q0 - hex8_across<0>(q0), u1 = q1 + g * hex8_across<0>(q1), u2 = q2 + g * hex8_across<0>(q2);
+  const R w0 = (u0 + g * hex8_across<1>(u0)) + (u1 - hex8_across<1>(u1)), w2 = u2 + g * hex8_across<1>(u2);
+  return (w0 + g * hex8_across<2>(w0)) + (w2 - hex8_across<2>(w2));
+}
+
+template <class R, int PH> constexpr int rows_hex8_waves() { return sizeof(R) == 4 ? 4 : PH == NEOHOOKE ? 2 : PH == THERMAL ? 3 : 5; }
+
+template <class R, int PH>
+__global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows_hex8(TArgs A) {
+  constexpr int N = 8, D = 3, P = PH == THERMAL ? 1 : 3;
+  using SH = RowsShape<HEX8, 2, N, P>;
+  constexpr int EB = 8, KW = SH::KW, OR = SH::OR, CPW = SH::CPW;
+  __shared__ __align__(16) R S[(64 + 4) * P * P];  // the lanes' blocks, column by column (4 of padding)
+  __shared__ unsigned long long MK[KW];
+  __shared__ int CS[KW + 1];
+  const int lane = threadIdx.x;
+  const long long per = gridDim.x / 8, rem = gridDim.x % 8;  // XCD x takes the x-th eighth of the nodes
+  const long long xcd = blockIdx.x % 8, qn = blockIdx.x / 8;
+  const long long node = xcd * per + (xcd < rem ? xcd : rem) + qn;
+  const int off0 = A.ne_off[node], cnt = A.ne_off[node + 1] - off0;
+  const long long rp = A.row_ptr[node * P];
+  const int deg = (int)((A.row_ptr[node * P + 1] - rp) / P);
+  bool dm[P], any_dm = false;
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    dm[c] = A.dmask[node * P + c] != 0;
+    any_dm = any_dm || dm[c];
+  }
+  const bool elemental = (A.flags & FEMHOT_ELEMENT_FIELD) != 0;
+  const bool accumulate = (A.flags & FEMHOT_ACCUMULATE) != 0;
+  const R *F = reinterpret_cast<const R *>(A.field);
+  const R *U = reinterpret_cast<const R *>(A.u);
+  R *V = reinterpret_cast<R *>(A.vals) + rp;
+  const int s = lane / 8, j = lane % 8, b = j < 4 ? j : 11 - j;  // the lane's node and Gauss point
+  const int ix = ((b & 3) == 1 || (b & 3) == 2) ? 1 : 0, iy = (b & 3) >= 2 ? 1 : 0, iz = b >= 4 ? 1 : 0;
+  const R sg[3] = {ix ? R(1) : R(-1), iy ? R(1) : R(-1), iz ? R(1) : R(-1)};
+  const int oc = lane / (CPW * P), kk = (lane - oc * CPW * P) / P, od = lane - oc * CPW * P - kk * P;
+  const R g = R(HEX8_G);
+  for (int k0 = 0; k0 < deg; k0 += KW) {
+    const int kw = min(KW, deg - k0);
+    R acc[OR];
+#pragma unroll
+    for (int r = 0; r < OR; ++r) acc[r] = R(0);
+    for (int base = 0; base < cnt; base += EB) {
+      const int nb = min(EB, cnt - base);
+      int a = 0, col = -1;
+      double xc[D] = {0.0, 0.0, 0.0};
+      R fd = R(0), ud[P];
+#pragma unroll
+      for (int c = 0; c < P; ++c) ud[c] = R(0);
+      if (s < nb) {
+        const int ea = A.ne_list[off0 + base + s];
+        const int e = ea / N;
+        a = ea - e * N;
+        col = A.slot[((size_t)e * N + a) * N + b];
+        const int nd = A.conn[(size_t)e * N + b];
+#pragma unroll
+        for (int i = 0; i < D; ++i) xc[i] = A.coords[(size_t)nd * 3 + i];
+        fd = elemental ? F[e] : F[nd];
+        if constexpr (PH != MECH) {
+#pragma unroll
+          for (int c = 0; c < P; ++c) ud[c] = U[(size_t)nd * P + c];
+        }
+      }
+      for (int t = lane; t < kw; t += 64) MK[t] = 0ull;
+      __syncthreads();
+      if (col >= k0 && col < k0 + kw) atomicOr(&MK[col - k0], 1ull << lane);
+      // J' = 8 J / (1 + s)^2 and its inverse
+      R J[D][D];
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        double ref = rows_dpp_into<0x150, 0x3>(xc[i], xc[i]);  // node 0 of the element
+        ref = rows_dpp_into<0x158, 0xc>(ref, xc[i]);
+        hex8_point_gradient<R>(R(xc[i] - ref), sg, J[i]);
+      }
+      const R c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
+      const R c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
+      const R c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
+      const R det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
+      const R id = recip(det);
+      R iv[D][D];
+      iv[0][0] = c00 * id;
+      iv[1][0] = c01 * id;
+      iv[2][0] = c02 * id;
+      iv[0][1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
+      iv[1][1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
+      iv[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
+      iv[0][2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
+      iv[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
+      iv[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
+      constexpr double a1 = 1.0 + HEX8_S, a3 = a1 * a1 * a1 / 8.0;
+      R f = R(a3 * a3 / 8.0) * det;  // det J = ((1 + s)^2 / 8)^3 det J'
+      f *= elemental ? fd : R(a3) * hex8_point_value<R>(fd);
+      // dN_a/dx of the owned node a (the factors of J' and of the shape gradients cancel)
+      const int ax = ((a & 3) == 1 || (a & 3) == 2) ? 1 : 0, ay = (a & 3) >= 2 ? 1 : 0, az = a >= 4 ? 1 : 0;
+      const R rx = ax == ix ? R(1) : g, ry = ay == iy ? R(1) : g, rz = az == iz ? R(1) : g;
+      const R sh[3] = {ax ? ry * rz : -(ry * rz), ay ? rx * rz : -(rx * rz), az ? rx * ry : -(rx * ry)};
+      R dNa[D];
+#pragma unroll
+      for (int q = 0; q < D; ++q) dNa[q] = (sh[0] * iv[0][q] + sh[1] * iv[1][q]) + sh[2] * iv[2][q];
+      R K[P * P];
+      if constexpr (PH == THERMAL) {
+        f *= R(1) + R(A.pp.beta) * powc(R(a3) * hex8_point_value<R>(ud[0]), R(A.pp.c));
+        R q[D];
+#pragma unroll
+        for (int k = 0; k < D; ++k) q[k] = (f * sg[k]) * ((dNa[0] * iv[k][0] + dNa[1] * iv[k][1]) + dNa[2] * iv[k][2]);
+        K[0] = hex8_node_sum<R>(q[0], q[1], q[2]);
+      } else if constexpr (PH == MECH) {
+        R fa[D], M[D][D];
+#pragma unroll
+        for (int i = 0; i < D; ++i) fa[i] = f * dNa[i];
+#pragma unroll
+        for (int q = 0; q < D; ++q) {
+          const R i0 = sg[0] * iv[0][q], i1 = sg[1] * iv[1][q], i2 = sg[2] * iv[2][q];
+#pragma unroll
+          for (int p = 0; p < D; ++p) M[p][q] = hex8_node_sum<R>(fa[p] * i0, fa[p] * i1, fa[p] * i2);
+        }
+        const R c2 = R(A.pp.c2), c3 = R(A.pp.c3), c4 = R(A.pp.c4);
+#pragma unroll
+        for (int c = 0; c < D; ++c)
+#pragma unroll
+          for (int d = 0; d < D; ++d)
+            K[c * P + d] = c == d ? c2 * M[c][c] + c4 * (M[(c + 1) % D][(c + 1) % D] + M[(c + 2) % D][(c + 2) % D])
+                                  : c3 * M[c][d] + c4 * M[d][c];
+      } else {
+        R H[D][D];
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+          R h[D];
+          hex8_point_gradient<R>(ud[i], sg, h);
+#pragma unroll
+          for (int q = 0; q < D; ++q) H[i][q] = (h[0] * iv[0][q] + h[1] * iv[1][q]) + h[2] * iv[2][q];
+        }
+        NHState<R, D> st;
+        nh_state<R, D>(H, R(A.pp.kap1), R(A.pp.mu1), st);
+        R Sa[D];  // S dN_a
+#pragma unroll
+        for (int i = 0; i < D; ++i) Sa[i] = (st.S[i][0] * dNa[0] + st.S[i][1] * dNa[1]) + st.S[i][2] * dNa[2];
+#pragma unroll
+        for (int c = 0; c < D; ++c) {  // the stress change of a unit displacement (a, c): F dS + dF S
+          R X[D][D], dS[D][D];
+#pragma unroll
+          for (int p = 0; p < D; ++p)
+#pragma unroll
+            for (int q = 0; q < D; ++q) X[p][q] = R(0.5) * (st.F[c][p] * dNa[q] + st.F[c][q] * dNa[p]);
+          nh_tangent_apply<R, D>(st, R(A.pp.kap1), R(A.pp.mu1), X, dS);
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            R w[D], q[D];
+#pragma unroll
+            for (int i = 0; i < D; ++i) {
+              const R m = (st.F[d][0] * dS[0][i] + st.F[d][1] * dS[1][i]) + st.F[d][2] * dS[2][i];
+              w[i] = f * (c == d ? m + Sa[i] : m);
+            }
+#pragma unroll
+            for (int k = 0; k < D; ++k) q[k] = sg[k] * ((w[0] * iv[k][0] + w[1] * iv[k][1]) + w[2] * iv[k][2]);
+            K[c * P + d] = hex8_node_sum<R>(q[0], q[1], q[2]);
+          }
+        }
+      }
+      if (any_dm) {  // a Dirichlet row keeps only the element diagonal (fe_loss.py:191-207)
+        asm volatile("" ::: "memory");  // keeps this a branch: the selects would run for every node
+#pragma unroll
+        for (int c = 0; c < P; ++c)
+#pragma unroll
+          for (int d = 0; d < P; ++d)
+            if (dm[c] && !(b == a && d == c)) K[c * P + d] = R(0);
+      }
+      __syncthreads();
+      rows_column_starts<KW>(lane, kw, MK, CS);
+      __syncthreads();
+      if (col >= k0 && col < k0 + kw) {
+        const int k = col - k0;
+        const int dst = CS[k] + __popcll(MK[k] & ((1ull << lane) - 1ull));
+#pragma unroll
+        for (int i = 0; i < P * P; ++i) S[dst * P * P + i] = K[i];
+      }
+      __syncthreads();
+      rows_add_columns<R, P, CPW, OR>(kw, oc, kk, od, S, CS, acc);
+      __syncthreads();  // before the next batch overwrites the blocks and the masks
+    }
+    rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
+  }
+}
+
+}  // namespace femhot
