@@ -346,7 +346,7 @@ class FemhotContext:
         return epc.value, blk.value, grid.value, ms.value
 
     def autotune_tangent(self, field, u, flags=0):
-        """Times atomic, colour-ordered and (thermal, linear elastic) row-owner tangent assembly on these
+        """Times atomic, colour-ordered and (where it covers the context) row-owner tangent assembly on these
         inputs and keeps the fastest for tangent_csr calls with SCATTER_CHUNK.  Returns (L.PATH_ATOMIC,
         L.PATH_COLOUR or L.PATH_ROWS, ms)."""
         field = field.reshape(-1).contiguous()

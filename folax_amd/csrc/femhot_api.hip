@@ -270,7 +270,7 @@ int femhot_tangent_csr(femhot_ctx *h, int dtype, const void *field, const void *
   hipStream_t s = (hipStream_t)stream;
   const bool acc = (flags & FEMHOT_ACCUMULATE) != 0;
   // FEMHOT_SCATTER_CHUNK leaves the assembly order to the library: the path femhot_autotune
-  // measured fastest for the tangent (untuned: row-owner, colour-ordered for Neo-Hookean)
+  // measured fastest for the tangent (untuned: row-owner, else colour-ordered)
   if ((flags & FEMHOT_SCATTER_CHUNK) && !(flags & (FEMHOT_SCATTER_COLOUR | FEMHOT_SCATTER_ROWS))) {
     const int path = tuned_path(c, dtype, MODE_TANGENT, 1, flags);
     if (path == PATH_COLOUR) flags |= FEMHOT_SCATTER_COLOUR;
@@ -311,7 +311,8 @@ int femhot_tangent_csr(femhot_ctx *h, int dtype, const void *field, const void *
     A.list = nullptr;
     A.count = c->Ne;
     L.grid = dim3((unsigned)c->Nn);
-    if (c->Nn && (rc = launch_tangent_any(c->et, L))) return rc;
+    A.R = R;  // formed beside the tangent
+    return c->Nn ? launch_tangent_any(c->et, L) : FEMHOT_OK;
   } else if ((flags & FEMHOT_SCATTER_COLOUR) && !c->repeated_nodes) {
     // colour-ordered plain adds need distinct nodes within an element (lanes of one element would
     // otherwise update the same entries); meshes with collapsed elements assemble with atomics

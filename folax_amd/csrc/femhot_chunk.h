@@ -39,7 +39,7 @@ constexpr int MODE_TANGENT = 3;
 // The path femhot_autotune measured fastest for this call shape; untuned: the chunk kernel, except
 // FP64 Neo-Hookean (its element routine needs most of the register file, so only small chunks with
 // small workgroups keep the chunk kernel ahead) which takes the atomic path, and the tangent, which
-// takes the row-owner assembly (colour-ordered adds for Neo-Hookean).
+// takes the row-owner assembly (colour-ordered adds where it does not cover the context).
 int tuned_path(const Ctx *c, int dtype, int mode, int batch, unsigned flags);
 
 // Records the path that won the autotuner for this call shape.

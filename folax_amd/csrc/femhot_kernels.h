@@ -75,6 +75,16 @@ __device__ __forceinline__ double wave_sum_to_last(double v) {
   return v;
 }
 
+__device__ __forceinline__ float wave_sum_to_last(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xa, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xc, 0xf, false));
+  return v;
+}
+
 // Sum `v` into energy[idx] with one atomic per wave when all active lanes share idx.
 __device__ __forceinline__ void add_energy(double *energy, int idx, double v, bool active) {
   const unsigned long long act = __ballot(active);
@@ -252,6 +262,7 @@ struct TArgs {
   const void *field;
   const void *u;
   void *vals;
+  void *R;  // row-owner assembly: the masked residual, or null
   const long long *row_ptr;
   const uint8_t *slot;
   const uint8_t *dmask;

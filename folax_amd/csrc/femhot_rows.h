@@ -22,6 +22,10 @@
 // which is B_a^T D B_b for the isotropic D of mechanical.py:60-82 (c2 = D_00, c3 = D_01, c4 = D_33 in
 // 3-D; f2, f2nu, f2sh of plane stress in 2-D).  Both element tangents are symmetric, so
 // FEMHOT_TRANSPOSE leaves them unchanged.
+//
+// Residual (A.R): formed in the same pass from the blocks, so a call that wants both reads the mesh and the
+// fields once and needs no second kernel, workspace or plan (HEX8 64^3 FP64, linear elastic: 495 us with the
+// residual through the chunk kernel, 447 here; 20^3: 47.9 and 37.8).
 #pragma once
 #include "femhot_kernels.h"
 
@@ -271,6 +275,22 @@ __device__ __forceinline__ void rows_write(int kw, int k0, int deg, int oc, int 
   }
 }
 
+// The owned node's residual from its lanes' shares (r: this lane's sum), masked as fe_loss.py:191-207: one
+// wave sum per component, the order fixed.
+template <class R, int P>
+__device__ __forceinline__ void rows_write_residual(const R (&r)[P], const bool (&dm)[P], bool accumulate, R *out) {
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    const R s = wave_sum_to_last(r[c]);
+    if ((threadIdx.x & 63) == 63) {
+      if (!accumulate)
+        out[c] = dm[c] ? R(0) : s;
+      else if (!dm[c])
+        out[c] += s;
+    }
+  }
+}
+
 // Waves per SIMD the compiler must fit: 3 for linear elasticity (168 VGPRs in FP64 HEX8 2x2x2, no spills);
 // the thermal instantiations keep the compiler's own choice (the powc of k(T) would spill under 3).
 template <int PH> constexpr int rows_min_waves() { return PH == MECH ? 3 : 1; }
@@ -326,7 +346,17 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
   // lane of the output stage: row oc, column kk of a round's CPW, component od (row by row, so a round
   // writes P runs of CPW * P values); lanes past P rows idle
   const int oc = lane / (CPW * P), kk = (lane - oc * CPW * P) / P, od = lane - oc * CPW * P - kk * P;
+  // The residual of these physics is K u (Picard K for thermal) less the body force, and the rows of K sum to
+  // zero, so with du_b = u_b - u_i it is sum K_ab du_b: 9 FMAs a lane beside the block that is formed anyway.
+  const bool want_r = A.R != nullptr;
+  R res[P], ui[P];
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    res[c] = R(0);
+    ui[c] = want_r ? U[node * P + c] : R(0);
+  }
   for (int k0 = 0; k0 < deg; k0 += KW) {
+    const bool first = want_r && k0 == 0;
     const int kw = min(KW, deg - k0);
     R acc[OR];
 #pragma unroll
@@ -336,6 +366,9 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       // 0. lane (s, b) fetches node b of incident element s: coordinates, field and (thermal)
       //    solution to LDS; its column among the owned node's neighbours stays in a register
       int a2 = 0, col = -1;
+      R du[P];
+#pragma unroll
+      for (int c = 0; c < P; ++c) du[c] = R(0);
       double xc[3] = {0.0, 0.0, 0.0};
       if (s2 < nb) {
         const int ea = A.ne_list[off0 + base + s2];
@@ -347,6 +380,10 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         for (int i = 0; i < 3; ++i) xc[i] = A.coords[(size_t)nd * 3 + i];
         FS[lane] = elemental ? F[e] : F[nd];
         if constexpr (PH == THERMAL) US[lane] = U[nd];
+        if (first) {
+#pragma unroll
+          for (int c = 0; c < P; ++c) du[c] = U[(size_t)nd * P + c] - ui[c];
+        }
       }
 #pragma unroll
       for (int i = 0; i < 3; ++i) XS[lane * 3 + i] = ET == HEX8 ? hex8_lane_moment(xc[i], b2) : xc[i];
@@ -359,6 +396,14 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         R *st = S + lane * ST;
         R Nv[N], inv[D][D];
         const R wdet = gp_inverse<R, ET, NGP>(g1, XS + n0 * 3, Nv, inv);
+        if (first && A.pp.has_body) {  // this lane's point of the owned node's body force
+          const int a1 = A.ne_list[off0 + base + s1] % N;
+          R na = Nv[0];
+#pragma unroll
+          for (int b = 1; b < N; ++b) na = b == a1 ? Nv[b] : na;
+#pragma unroll
+          for (int c = 0; c < P; ++c) res[c] -= (wdet * na) * R(A.pp.body[c]);
+        }
         R eg;
         if (elemental) {
           eg = FS[n0];
@@ -444,6 +489,12 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
               }
             }
         }
+        if (first && s2 < nb) {
+#pragma unroll
+          for (int c = 0; c < P; ++c)
+#pragma unroll
+            for (int d = 0; d < P; ++d) res[c] += K[c * P + d] * du[d];
+        }
         // a Dirichlet row keeps only the element diagonal (fe_loss.py:191-207); dm is the same for
         // the whole workgroup, so free nodes skip this
         if (any_dm) {
@@ -468,6 +519,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
     }
     rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
   }
+  if (want_r) rows_write_residual<R, P>(res, dm, accumulate, reinterpret_cast<R *>(A.R) + node * P);
 }
 
 }  // namespace femhot

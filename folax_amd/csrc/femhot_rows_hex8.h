@@ -14,7 +14,9 @@
 // per SIMD), and each of the blocks' 9 entries costs 26 instructions.  A lane's partners are lane ^ 1, ^ 3
 // and ^ 7, one DPP move per 32 bits: lanes 4..7 hold the upper nodes in the order 7, 6, 5, 4.
 //
-// Bound: FP64 vector issue.  MEASURED
+// Bound: FP64 vector issue.  HEX8 64^3 FP64, tangent and residual of the linear-elastic box: 669 us through
+// the general kernel (its tangent 565), 495 with the butterflies and the residual through the chunk
+// kernel, 447 with the residual formed here.
 #pragma once
 #include "femhot_rows.h"
 
@@ -86,7 +88,17 @@ __global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows
   const R sg[3] = {ix ? R(1) : R(-1), iy ? R(1) : R(-1), iz ? R(1) : R(-1)};
   const int oc = lane / (CPW * P), kk = (lane - oc * CPW * P) / P, od = lane - oc * CPW * P - kk * P;
   const R g = R(HEX8_G);
+  // The residual beside the tangent: sum K_ab (u_b - u_i) for the linear physics (see femhot_rows.h), the
+  // stress times dN_a at the lane's point for Neo-Hookean, less the body force N_a b at that point.
+  const bool want_r = A.R != nullptr;
+  R res[P], ui[P];
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    res[c] = R(0);
+    ui[c] = want_r ? U[node * P + c] : R(0);
+  }
   for (int k0 = 0; k0 < deg; k0 += KW) {
+    const bool first = want_r && k0 == 0;
     const int kw = min(KW, deg - k0);
     R acc[OR];
 #pragma unroll
@@ -107,7 +119,7 @@ __global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows
 #pragma unroll
         for (int i = 0; i < D; ++i) xc[i] = A.coords[(size_t)nd * 3 + i];
         fd = elemental ? F[e] : F[nd];
-        if constexpr (PH != MECH) {
+        if (PH != MECH || first) {
 #pragma unroll
           for (int c = 0; c < P; ++c) ud[c] = U[(size_t)nd * P + c];
         }
@@ -139,8 +151,8 @@ __global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows
       iv[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
       iv[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
       constexpr double a1 = 1.0 + HEX8_S, a3 = a1 * a1 * a1 / 8.0;
-      R f = R(a3 * a3 / 8.0) * det;  // det J = ((1 + s)^2 / 8)^3 det J'
-      f *= elemental ? fd : R(a3) * hex8_point_value<R>(fd);
+      const R wdet = R(a3 * a3 / 8.0) * det;  // det J = ((1 + s)^2 / 8)^3 det J'
+      R f = wdet * (elemental ? fd : R(a3) * hex8_point_value<R>(fd));
       // dN_a/dx of the owned node a (the factors of J' and of the shape gradients cancel)
       const int ax = ((a & 3) == 1 || (a & 3) == 2) ? 1 : 0, ay = (a & 3) >= 2 ? 1 : 0, az = a >= 4 ? 1 : 0;
       const R rx = ax == ix ? R(1) : g, ry = ay == iy ? R(1) : g, rz = az == iz ? R(1) : g;
@@ -186,6 +198,11 @@ __global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows
         R Sa[D];  // S dN_a
 #pragma unroll
         for (int i = 0; i < D; ++i) Sa[i] = (st.S[i][0] * dNa[0] + st.S[i][1] * dNa[1]) + st.S[i][2] * dNa[2];
+        if (first && s < nb) {
+#pragma unroll
+          for (int c = 0; c < D; ++c)
+            res[c] += f * ((st.F[c][0] * Sa[0] + st.F[c][1] * Sa[1]) + st.F[c][2] * Sa[2]);
+        }
 #pragma unroll
         for (int c = 0; c < D; ++c) {  // the stress change of a unit displacement (a, c): F dS + dF S
           R X[D][D], dS[D][D];
@@ -206,6 +223,19 @@ __global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows
             for (int k = 0; k < D; ++k) q[k] = sg[k] * ((w[0] * iv[k][0] + w[1] * iv[k][1]) + w[2] * iv[k][2]);
             K[c * P + d] = hex8_node_sum<R>(q[0], q[1], q[2]);
           }
+        }
+      }
+      if (first && s < nb) {
+        if constexpr (PH != NEOHOOKE) {
+#pragma unroll
+          for (int c = 0; c < P; ++c)
+#pragma unroll
+            for (int d = 0; d < P; ++d) res[c] += K[c * P + d] * (ud[d] - ui[d]);
+        }
+        if (A.pp.has_body) {
+          const R na = R(a3) * wdet * (rx * (ry * rz));
+#pragma unroll
+          for (int c = 0; c < P; ++c) res[c] -= na * R(A.pp.body[c]);
         }
       }
       if (any_dm) {  // a Dirichlet row keeps only the element diagonal (fe_loss.py:191-207)
@@ -231,6 +261,7 @@ __global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows
     }
     rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
   }
+  if (want_r) rows_write_residual<R, P>(res, dm, accumulate, reinterpret_cast<R *>(A.R) + node * P);
 }
 
 }  // namespace femhot

@@ -62,7 +62,8 @@ extern "C" {
 #define FEMHOT_SCATTER_COLOUR 0x20u /* colour-ordered, non-atomic, deterministic scatter */
 #define FEMHOT_SCATTER_CHUNK 0x40u  /* LDS-staged chunk scatter (persistent launch) */
 #define FEMHOT_SCATTER_ROWS 0x80u   /* tangent: row-owner assembly, each CSR value summed in a fixed
-                                       order and written once (thermal, linear elastic) */
+                                       order and written once (thermal, linear elastic,
+                                       Neo-Hookean on 2x2x2 HEX8) */
 
 /* status codes */
 #define FEMHOT_OK 0
@@ -125,10 +126,10 @@ int femhot_residual(femhot_ctx *ctx, int dtype, int batch, const void *field, lo
  * fe_loss.py:191-207; FEMHOT_TRANSPOSE transposes each element matrix first.  Assembly: hardware
  * atomics into zero-filled values (no scatter flag), colour-ordered plain adds
  * (FEMHOT_SCATTER_COLOUR), or row-owner assembly (FEMHOT_SCATTER_ROWS: one workgroup per node sums
- * the node's rows from its incident elements in element order and writes each value once; no fill,
- * deterministic; thermal and linear elastic, Neo-Hookean falls back to colour-ordered adds);
- * FEMHOT_SCATTER_CHUNK takes the one femhot_autotune measured fastest (untuned: row-owner, for
- * Neo-Hookean colour-ordered). */
+ * the node's rows from its incident elements in element order and writes each value once, the residual
+ * with them; no fill, deterministic; Neo-Hookean on other elements and rules than 2x2x2 HEX8 falls back
+ * to colour-ordered adds); FEMHOT_SCATTER_CHUNK takes the one femhot_autotune measured fastest
+ * (untuned: row-owner, else colour-ordered). */
 int femhot_tangent_csr(femhot_ctx *ctx, int dtype, const void *field, const void *u, void *vals, void *R,
                        unsigned flags, void *stream);
 
