@@ -312,6 +312,8 @@ int femhot_tangent_csr(femhot_ctx *h, int dtype, const void *field, const void *
     A.count = c->Ne;
     L.grid = dim3((unsigned)c->Nn);
     A.R = R;  // formed beside the tangent
+    A.r2 = c->pp.c4 != 0.0 ? (c->pp.c2 - c->pp.c4) / c->pp.c4 : 0.0;  // (c4 = 0 only with E = 0: K = 0)
+    A.r3 = c->pp.c4 != 0.0 ? c->pp.c3 / c->pp.c4 : 0.0;
     return c->Nn ? launch_tangent_any(c->et, L) : FEMHOT_OK;
   } else if ((flags & FEMHOT_SCATTER_COLOUR) && !c->repeated_nodes) {
     // colour-ordered plain adds need distinct nodes within an element (lanes of one element would

@@ -55,10 +55,16 @@ template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_f64(double v
   return __hiloint2double(hi, lo);
 }
 
-// v of the lane that DPP control CTRL names (every lane has one).
-template <int CTRL> __device__ __forceinline__ double lane_dpp(double v) { return dpp_f64<CTRL, 0xf>(v); }
-template <int CTRL> __device__ __forceinline__ float lane_dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+// v of the lane that DPP control CTRL names, in the banks of BANKS; the others are undefined.  (Every lane
+// named must be active.  A move without an old value costs one instruction per 32 bits; one that keeps
+// an old value costs two, for it is first copied into the destination.)
+template <int CTRL, int BANKS = 0xf> __device__ __forceinline__ double lane_dpp(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, BANKS, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, BANKS, true);
+  return __hiloint2double(hi, lo);
+}
+template <int CTRL, int BANKS = 0xf> __device__ __forceinline__ float lane_dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, BANKS, true));
 }
 
 // Sum over the 64 lanes of a wave, valid in lane 63 only: pairs and quads (quad_perm), half rows and
@@ -66,20 +72,20 @@ template <int CTRL> __device__ __forceinline__ float lane_dpp(float v) {
 // rows 0-1 into rows 2-3 (row_bcast:31).  Register moves instead of the LDS round trips of a shuffle
 // butterfly; a fixed order, so the sum is the same on every run.
 __device__ __forceinline__ double wave_sum_to_last(double v) {
-  v += dpp_f64<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f64<0x4E, 0xf>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f64<0x141, 0xf>(v);  // row_half_mirror
-  v += dpp_f64<0x140, 0xf>(v);  // row_mirror
+  v += lane_dpp<0xB1>(v);       // quad_perm [1,0,3,2]
+  v += lane_dpp<0x4E>(v);       // quad_perm [2,3,0,1]
+  v += lane_dpp<0x141>(v);      // row_half_mirror
+  v += lane_dpp<0x140>(v);      // row_mirror
   v += dpp_f64<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
   v += dpp_f64<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
   return v;
 }
 
 __device__ __forceinline__ float wave_sum_to_last(float v) {
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false));
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false));
+  v += lane_dpp<0xB1>(v);
+  v += lane_dpp<0x4E>(v);
+  v += lane_dpp<0x141>(v);
+  v += lane_dpp<0x140>(v);
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xa, 0xf, false));
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xc, 0xf, false));
   return v;
@@ -268,6 +274,7 @@ struct TArgs {
   const uint8_t *dmask;
   const int *ne_off, *ne_list;  // row-owner assembly: node -> (element * n + local index)
   long long n_nodes;
+  double r2, r3;  // linear elasticity, HEX8 rows: (c2 - c4) / c4 and c3 / c4
   unsigned flags;
   PhysParams pp;
 };

@@ -207,15 +207,15 @@ template <int CTRL, int BANKS> __device__ __forceinline__ double rows_dpp_into(d
 }
 __device__ __forceinline__ double hex8_lane_moment(double v, int b) {
   // node 0's value: lane 0 of the lower and lane 8 of the upper half of each row of 16 (row_newbcast)
-  double ref = rows_dpp_into<0x150, 0x3>(v, v);
+  double ref = lane_dpp<0x150, 0x3>(v);
   ref = rows_dpp_into<0x158, 0xc>(ref, v);
   v -= ref;
   const double sx = (b & 3) == 1 || (b & 3) == 2 ? -1.0 : 1.0, sy = (b & 3) >= 2 ? -1.0 : 1.0, sz = b >= 4 ? -1.0 : 1.0;
   // the lane on the - side adds its partner, the one on the + side subtracts it (products by +-1 are exact)
-  v = __builtin_fma(sx, rows_dpp_into<0xB1, 0xf>(0.0, v), v);  // b ^ 1 (quad_perm [1,0,3,2])
-  v = __builtin_fma(sy, rows_dpp_into<0x1B, 0xf>(0.0, v), v);  // b ^ 3 (quad_perm [3,2,1,0])
-  double up = rows_dpp_into<0x104, 0x5>(0.0, v);               // b ^ 4: row_shl:4 into banks 0 and 2,
-  up = rows_dpp_into<0x114, 0xa>(up, v);                       // row_shr:4 into banks 1 and 3
+  v = __builtin_fma(sx, lane_dpp<0xB1>(v), v);  // b ^ 1 (quad_perm [1,0,3,2])
+  v = __builtin_fma(sy, lane_dpp<0x1B>(v), v);  // b ^ 3 (quad_perm [3,2,1,0])
+  double up = lane_dpp<0x104, 0x5>(v);    // b ^ 4: row_shl:4 into banks 0 and 2,
+  up = rows_dpp_into<0x114, 0xa>(up, v);  // row_shr:4 into banks 1 and 3
   return __builtin_fma(sz, up, v);
 }
 
@@ -242,23 +242,51 @@ __device__ __forceinline__ void rows_column_starts(int lane, int kw, const unsig
 }
 
 // Output stage: a lane owns row oc, component od and column kk of each round's CPW, and adds the column's
-// blocks in lane order (S reaches 3 blocks past the last).
+// blocks in lane order.  The first four blocks of every round are loaded together, so their LDS latency is
+// paid once and not once a round (S reaches 3 blocks past the last); the sums stop at the column's end
+// by branches, for a select costs three instructions an entry.
+template <class R, int N> __device__ __forceinline__ R rows_sum_four(int n, const R (&x)[N], R sum) {
+  if (n > 0) {
+    sum += x[0];
+    if (n > 1) {
+      asm volatile("" ::: "memory");  // keeps these branches
+      sum += x[1];
+      if (n > 2) {
+        asm volatile("" ::: "memory");
+        sum += x[2];
+        if (n > 3) {
+          asm volatile("" ::: "memory");
+          sum += x[3];
+        }
+      }
+    }
+  }
+  return sum;
+}
 template <class R, int P, int CPW, int OR>
 __device__ __forceinline__ void rows_add_columns(int kw, int oc, int kk, int od, const R *S, const int *CS,
                                                  R (&acc)[OR]) {
+  int lo[OR], n[OR];
+  R x[OR][4];
 #pragma unroll
   for (int r = 0; r < OR; ++r) {
     const int k = r * CPW + kk;
-    if (k >= kw || oc >= P) continue;
-    const int lo = CS[k], hi = CS[k + 1];
-    R sum = R(0);
-    for (int i = lo; i < hi; i += 4) {  // four contributions per round, their loads issued together
-      const R *src = S + i * (P * P) + oc * P + od;
-      R x[4];
+    const bool own = k < kw && oc < P;
+    lo[r] = own ? CS[k] : 0;
+    n[r] = own ? CS[k + 1] - lo[r] : 0;
+  }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) x[q] = src[q * P * P];
+  for (int r = 0; r < OR; ++r)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) sum += (i + q < hi) ? x[q] : R(0);
+    for (int q = 0; q < 4; ++q) x[r][q] = S[(lo[r] + q) * (P * P) + oc * P + od];
+#pragma unroll
+  for (int r = 0; r < OR; ++r) {
+    R sum = rows_sum_four(n[r], x[r], R(0));
+    for (int i = 4; i < n[r]; i += 4) {
+      R y[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) y[q] = S[(lo[r] + i + q) * (P * P) + oc * P + od];
+      sum = rows_sum_four(n[r] - i, y, sum);
     }
     acc[r] += sum;
   }
@@ -275,19 +303,48 @@ __device__ __forceinline__ void rows_write(int kw, int k0, int deg, int oc, int 
   }
 }
 
-// The owned node's residual from its lanes' shares (r: this lane's sum), masked as fe_loss.py:191-207: one
-// wave sum per component, the order fixed.
-template <class R, int P>
-__device__ __forceinline__ void rows_write_residual(const R (&r)[P], const bool (&dm)[P], bool accumulate, R *out) {
+// K (u - u_i) of the output lanes' values of one window: DU = the columns' u_b - u_i.
+template <class R, int P, int CPW, int OR>
+__device__ __forceinline__ R rows_apply(int kw, int oc, int kk, int od, const R *DU, const R (&acc)[OR]) {
+  R s = R(0);
 #pragma unroll
-  for (int c = 0; c < P; ++c) {
-    const R s = wave_sum_to_last(r[c]);
-    if ((threadIdx.x & 63) == 63) {
-      if (!accumulate)
-        out[c] = dm[c] ? R(0) : s;
-      else if (!dm[c])
-        out[c] += s;
+  for (int r = 0; r < OR; ++r) {
+    const int k = r * CPW + kk;
+    if (k < kw && oc < P) s += acc[r] * DU[k * P + od];
+  }
+  return s;
+}
+
+// The owned node's residual, masked as fe_loss.py:191-207: the output lanes' shares of K (u - u_i) (SHARES;
+// lane / G is the component) and, with lanes, each lane's own res, summed in a fixed order.  S: 64 values of scratch.
+template <class R, int P, int G, bool SHARES>
+__device__ __forceinline__ void rows_write_residual(R share, const R (&res)[P], bool lanes, unsigned dm,
+                                                    bool accumulate, R *S, R *out) {
+  const int lane = threadIdx.x, c = lane >> 4;  // 16 lanes per component
+  R x = R(0);
+  if constexpr (SHARES) {
+    S[lane] = share;
+    __syncthreads();
+    for (int m = lane & 15; c < P && m < G; m += 16) x += S[c * G + m];
+    x += lane_dpp<0xB1>(x);
+    x += lane_dpp<0x4E>(x);
+    x += lane_dpp<0x141>(x);
+    x += lane_dpp<0x140>(x);
+    __syncthreads();
+  }
+  const bool masked = (dm >> c) & 1;
+  if (lanes) {
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+      const R s = __shfl(wave_sum_to_last(res[k]), 63);
+      x += c == k ? s : R(0);
     }
+  }
+  if ((lane & 15) == 0 && c < P) {
+    if (!accumulate)
+      out[c] = masked ? R(0) : x;
+    else if (!masked)
+      out[c] += x;
   }
 }
 
@@ -317,6 +374,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
   __shared__ __align__(16) R S[SX];
   __shared__ unsigned long long MK[KW];
   __shared__ int CS[KW + 1];
+  __shared__ R DU[KW * P];  // u_b - u_i of the window's columns
   double *XS = reinterpret_cast<double *>(S + SX - XW);
   R *FS = reinterpret_cast<R *>(XS + 64 * 3);
   R *US = FS + 64;
@@ -330,12 +388,9 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
   const int off0 = A.ne_off[node], cnt = A.ne_off[node + 1] - off0;
   const long long rp = A.row_ptr[node * P];
   const int deg = (int)((A.row_ptr[node * P + 1] - rp) / P);
-  bool dm[P];
-#pragma unroll
-  for (int c = 0; c < P; ++c) dm[c] = A.dmask[node * P + c] != 0;
-  bool any_dm = false;
-#pragma unroll
-  for (int c = 0; c < P; ++c) any_dm = any_dm || dm[c];
+  // the Dirichlet mask in lanes 0..P-1, a bit mask where it is needed (read as a scalar it would be waited
+  // for before the first element is fetched)
+  const int dmv = lane < P ? A.dmask[node * P + lane] : 0;
   const bool elemental = (A.flags & FEMHOT_ELEMENT_FIELD) != 0;
   const bool accumulate = (A.flags & FEMHOT_ACCUMULATE) != 0;
   const R *F = reinterpret_cast<const R *>(A.field);
@@ -347,9 +402,9 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
   // writes P runs of CPW * P values); lanes past P rows idle
   const int oc = lane / (CPW * P), kk = (lane - oc * CPW * P) / P, od = lane - oc * CPW * P - kk * P;
   // The residual of these physics is K u (Picard K for thermal) less the body force, and the rows of K sum to
-  // zero, so with du_b = u_b - u_i it is sum K_ab du_b: 9 FMAs a lane beside the block that is formed anyway.
+  // zero, so with du_b = u_b - u_i it is sum K_ab du_b: an FMA per value in the output lanes.
   const bool want_r = A.R != nullptr;
-  R res[P], ui[P];
+  R res[P], ui[P], share = R(0);
 #pragma unroll
   for (int c = 0; c < P; ++c) {
     res[c] = R(0);
@@ -366,9 +421,6 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       // 0. lane (s, b) fetches node b of incident element s: coordinates, field and (thermal)
       //    solution to LDS; its column among the owned node's neighbours stays in a register
       int a2 = 0, col = -1;
-      R du[P];
-#pragma unroll
-      for (int c = 0; c < P; ++c) du[c] = R(0);
       double xc[3] = {0.0, 0.0, 0.0};
       if (s2 < nb) {
         const int ea = A.ne_list[off0 + base + s2];
@@ -380,9 +432,9 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         for (int i = 0; i < 3; ++i) xc[i] = A.coords[(size_t)nd * 3 + i];
         FS[lane] = elemental ? F[e] : F[nd];
         if constexpr (PH == THERMAL) US[lane] = U[nd];
-        if (first) {
+        if (want_r && col >= k0 && col < k0 + kw) {
 #pragma unroll
-          for (int c = 0; c < P; ++c) du[c] = U[(size_t)nd * P + c] - ui[c];
+          for (int c = 0; c < P; ++c) DU[(col - k0) * P + c] = U[(size_t)nd * P + c] - ui[c];
         }
       }
 #pragma unroll
@@ -438,9 +490,8 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         stage_gradients<R, ET, NGP>(go, iv, st);
       }
       __syncthreads();
-      {  // blocks are stored column by column, lanes in order: CS[k] = first block of column k
-        rows_column_starts<KW>(lane, kw, MK, CS);
-      }
+      rows_column_starts<KW>(lane, kw, MK, CS);  // blocks are stored column by column, lanes in order
+      const unsigned dm = (unsigned)__ballot(dmv != 0);
       R K[P * P];
       {  // 2. block (a, b) of each incident element's tangent (lanes past the batch's elements form one that
          // is not stored, from whatever their slots hold)
@@ -489,21 +540,15 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
               }
             }
         }
-        if (first && s2 < nb) {
-#pragma unroll
-          for (int c = 0; c < P; ++c)
-#pragma unroll
-            for (int d = 0; d < P; ++d) res[c] += K[c * P + d] * du[d];
-        }
         // a Dirichlet row keeps only the element diagonal (fe_loss.py:191-207); dm is the same for
         // the whole workgroup, so free nodes skip this
-        if (any_dm) {
+        if (dm) {
           asm volatile("" ::: "memory");  // keeps this a branch: the selects would run for every node
 #pragma unroll
           for (int c = 0; c < P; ++c)
 #pragma unroll
             for (int d = 0; d < P; ++d)
-              if (dm[c] && !(b == a && d == c)) K[c * P + d] = R(0);
+              if ((dm >> c & 1) && !(b == a && d == c)) K[c * P + d] = R(0);
         }
       }
       __syncthreads();  // every lane has read the staged geometry: the space takes the blocks
@@ -518,8 +563,12 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       __syncthreads();  // before the next batch overwrites the blocks and the masks
     }
     rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
+    if (want_r) share += rows_apply<R, P, CPW, OR>(kw, oc, kk, od, DU, acc);
+    __syncthreads();  // before the next window's DU
   }
-  if (want_r) rows_write_residual<R, P>(res, dm, accumulate, reinterpret_cast<R *>(A.R) + node * P);
+  if (want_r)
+    rows_write_residual<R, P, CPW * P, true>(share, res, A.pp.has_body, (unsigned)__ballot(dmv != 0), accumulate, S,
+                                             reinterpret_cast<R *>(A.R) + node * P);
 }
 
 }  // namespace femhot
