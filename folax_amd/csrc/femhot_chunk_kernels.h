@@ -104,13 +104,15 @@ template <class R, int K> __device__ __forceinline__ void store_corner_results(R
 //   ERD [emax * N + cap4 * pad]  per element corner, at the same row: nodal field-gradient contribution
 // Waves per SIMD the compiler must fit: 4 for FP32 TET4 thermal and linear elasticity at 256 threads
 // (their LDS holds 4 workgroups of 512-tet chunks per CU, so more registers would only cost waves),
-// else its own choice.
-template <class R, int ET, int PH, int BLOCK> constexpr int chunk_min_waves() {
+// 3 for the FP32 HEX8 Neo-Hookean residual (8 spilled registers; a 48^3 x 16 loss and
+// gradient: 300 -> 265 us; the gradient of the potential spills 20 and loses 4 %), else its own choice.
+template <class R, int ET, int PH, int MODE, int BLOCK> constexpr int chunk_min_waves() {
+  if (sizeof(R) == 4 && ET == HEX8 && PH == NEOHOOKE && MODE == MODE_RES && BLOCK <= 256) return 3;
   return (sizeof(R) == 4 && ET == TET4 && PH != NEOHOOKE && BLOCK == 256) ? 4 : 1;
 }
 
 template <class R, int ET, int PH, int NGP, int MODE, int BLOCK>
-__global__ __launch_bounds__(BLOCK, (chunk_min_waves<R, ET, PH, BLOCK>())) void k_chunk(ChunkArgs A) {
+__global__ __launch_bounds__(BLOCK, (chunk_min_waves<R, ET, PH, MODE, BLOCK>())) void k_chunk(ChunkArgs A) {
   using E = Elem<R, ET, PH>;
   constexpr int N = E::N, D = E::D, P = E::P, NL = E::NL;
   // nodes / elements per lane per round of loads: enough that one round covers 512 nodes and

