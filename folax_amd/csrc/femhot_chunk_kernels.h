@@ -102,6 +102,36 @@ template <class R, int K> __device__ __forceinline__ void store_corner_results(R
 //                       (the plan's rank of the corner) + pad * chunk node][component], so each node's
 //                       corners are one contiguous run
 //   ERD [emax * N + cap4 * pad]  per element corner, at the same row: nodal field-gradient contribution
+// s += the P-vectors lo .. hi - 1 of E (LDS) in order.  Four are loaded before the first is added: one at a
+// time, a node's sum pays the LDS latency once per corner, the longest serial chain of the kernel (24 corners
+// for an interior node of a tetrahedral mesh).  The last, partial four re-read the last corner and add -0,
+// which changes no sum.  (32 tetrahedral meshes, potential and gradient in FP32: 90.3 -> 89.2 us; the waves of a CU
+// had hidden most of it.)
+template <class R, int P> __device__ __forceinline__ void sum_corners(const R *E, int lo, int hi, R (&s)[P]) {
+  R x[4][P];
+  int j = lo;
+  for (; j + 4 <= hi; j += 4) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int c = 0; c < P; ++c) x[q][c] = E[(j + q) * P + c];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int c = 0; c < P; ++c) s[c] += x[q][c];
+  }
+  if (j < hi) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int c = 0; c < P; ++c) x[q][c] = E[min(j + q, hi - 1) * P + c];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int c = 0; c < P; ++c) s[c] += j + q < hi ? x[q][c] : R(-0.0);
+  }
+}
+
 // Waves per SIMD the compiler must fit: 4 for FP32 TET4 thermal and linear elasticity at 256 threads
 // (their LDS holds 4 workgroups of 512-tet chunks per CU, so more registers would only cost waves),
 // 3 for the FP32 HEX8 Neo-Hookean residual (8 spilled registers; a 48^3 x 16 loss and
@@ -384,11 +414,7 @@ __global__ __launch_bounds__(BLOCK, (chunk_min_waves<R, ET, PH, MODE, BLOCK>()))
 #pragma unroll
               for (int c = 0; c < P; ++c) s[c] = R(-0.0);
               // the node's corner results lie at its list positions js .. je - 1 (+ i with the spare rows)
-              for (int j = js[k] + pad * i; j < je[k] + pad * i; ++j) {
-                const R *e = ER + j * P;
-#pragma unroll
-                for (int c = 0; c < P; ++c) s[c] += e[c];
-              }
+              sum_corners<R, P>(ER, js[k] + pad * i, je[k] + pad * i, s);
               if (sl[k] >= 0) {  // a shared node: its partial slot, the P values stored back to back
                 R *pu = PU + (long long)sl[k] * P;
 #pragma unroll
@@ -408,14 +434,14 @@ __global__ __launch_bounds__(BLOCK, (chunk_min_waves<R, ET, PH, MODE, BLOCK>()))
               }
             }
             if (nodal_gd) {
-              R s = R(0);
-              for (int j = js[k] + pad * i; j < je[k] + pad * i; ++j) s += ERD[j];
+              R s[1] = {R(0)};
+              sum_corners<R, 1>(ERD, js[k] + pad * i, je[k] + pad * i, s);
               if (sl[k] >= 0)
-                PD[sl[k]] = s;
+                PD[sl[k]] = s[0];
               else if (accumulate)
-                unsafeAtomicAdd(&ODb[g[k]], s);
+                unsafeAtomicAdd(&ODb[g[k]], s[0]);
               else
-                ODb[g[k]] = s;
+                ODb[g[k]] = s[0];
             }
           }
         }
