@@ -19,9 +19,11 @@
 // coordinates.  HEX8 64^3 FP64, tangent and residual of the linear-elastic box with its boundary
 // conditions: 669 us through the general kernel (its tangent 565), 495 with the butterflies and the residual
 // through the chunk kernel, 447 with the residual formed here, 405 with lane moves that keep no old
-// value, 397 with the signs, the determinant and c4 taken out of the butterflies, the residual summed in the
+// value, 392 with the signs, the determinant and c4 taken out of the butterflies, the residual summed in the
 // output lanes and the list of blocks found while the coordinates arrive.  A loop over nodes in a wave with the next
-// node's connectivity fetched ahead was slower (484: its registers leave 3 waves per SIMD).
+// node's connectivity fetched ahead was slower (484: its registers leave 3 waves per SIMD).  The values are
+// stored after the residual's shares are formed (389).
+// The residual is 35 us of the 389.
 #pragma once
 #include "femhot_rows.h"
 
@@ -270,11 +272,11 @@ __global__ __launch_bounds__(64, (rows_hex8_waves<R, PH>())) void k_tangent_rows
       rows_add_columns<R, P, CPW, OR>(kw, oc, kk, od, S, CS, acc);
       __syncthreads();  // before the next batch overwrites the blocks and the masks
     }
-    rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
     if constexpr (PH != NEOHOOKE) {
       if (want_r) share += rows_apply<R, P, CPW, OR>(kw, oc, kk, od, DU, acc);
       __syncthreads();  // before the next window's DU
     }
+    rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
   }
   if (want_r)
     rows_write_residual<R, P, CPW * P, PH != NEOHOOKE>(share, res, PH == NEOHOOKE || A.pp.has_body,
