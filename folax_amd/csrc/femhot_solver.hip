@@ -502,6 +502,24 @@ template <class T> static size_t tile_ws_bytes(const Ctx *c, const TilePlan &tp)
   return 2 * r256(sizeof(T) * c->Ndof) + r256(sizeof(double) * 8 * tp.G) + 2 * r256(sizeof(PcgState));
 }
 
+// Workspace of an FP64 solve on this context, host-checked or enqueued, on the context's pattern or any
+// other: the most that any of their forms takes, so the first call of one kind sizes it for all of them and a
+// later call of another kind neither allocates under a capture nor frees what a captured graph uses.  Each
+// piece is 256-byte aligned.
+static size_t pcg_ws_bytes(const Ctx *c) {
+  const size_t vec64 = r256(sizeof(double) * c->Ndof), state = r256(sizeof(PcgState));
+  size_t need = 0;
+  for (const bool node_blocked : {false, true}) {  // launched: partials, 5 vectors, the state
+    const size_t nsp = spmv_plan(c->Ndof, c->nnz, c->ndpn, node_blocked).blocks;
+    need = std::max(need, r256(3 * NBR * sizeof(double)) + r256(NBR * sizeof(double)) + r256(nsp * sizeof(double)) +
+                              r256(8 * sizeof(double)) + 5 * vec64 + state);
+  }
+  const TilePlan tp = tile_plan<double>(c);
+  if (tp.ok)  // in one launch; one launch per phase: 6 vectors, partials, the state
+    need = std::max({need, tile_ws_bytes<double>(c, tp), 6 * vec64 + r256(sizeof(double) * 8 * tp.G) + state});
+  return need;
+}
+
 // One resident solve (k_pcg_resident), synchronised: *st the final state; *ran false when it could not be
 // launched or a wait between its workgroups ran out (x is then untouched).
 template <class T>
@@ -670,21 +688,19 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
   const long long n = c->Ndof, nnz = c->nnz;
   const dim3 grid((unsigned)((n + 255) / 256));
   const int check = 10;
-  // workspace: reduction partials (5 x NBR doubles) + 5 FP64 vectors + (FP32 mode) 5 FP32 vectors + FP32 matrix
   const size_t vec64 = sizeof(double) * n, vec32 = sizeof(float) * n;
   const SpmvPlan sp = spmv_plan(n, nnz, c->ndpn, node_blocked);
   const size_t nsp = sp.blocks;
-  size_t need = (4 * NBR + nsp + 8) * sizeof(double) + 1024 + 5 * vec64 + 1024;
-  if (mode == FEMHOT_F32) need += 5 * vec32 + sizeof(float) * nnz + 1024;
   // systems the tile kernels hold are solved in one launch (mixed: one launch per inner solve)
   TilePlan tp;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   FH_HIP(hipStreamIsCapturing(s, &cs));
   if (node_blocked && cs == hipStreamCaptureStatusNone)
     tp = mode == FEMHOT_F64 ? tile_plan<double>(c) : tile_plan<float>(c);
-  const size_t tile_bytes = !tp.ok ? 0 : mode == FEMHOT_F64 ? tile_ws_bytes<double>(c, tp) : tile_ws_bytes<float>(c, tp);
-  need = std::max(need, tile_bytes) + (mode == FEMHOT_F32 ? tile_bytes : 0);
-  rc = ensure_workspace(c, need);
+  // FP32 mode keeps an FP32 matrix and 5 FP32 vectors, and the resident solve's buffers, beside the FP64 part
+  const size_t tile_bytes = mode == FEMHOT_F32 && tp.ok ? tile_ws_bytes<float>(c, tp) : 0;
+  rc = ensure_workspace(c, pcg_ws_bytes(c) + (mode == FEMHOT_F32 ? tile_bytes + 5 * r256(vec32) + r256(sizeof(float) * nnz)
+                                                                 : 0));
   if (rc) return rc;
   if (tp.ok && mode == FEMHOT_F64) {
     PcgState st{};
@@ -809,19 +825,6 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
   return FEMHOT_OK;
 }
 
-// Workspace of femhot_pcg_async: the layout of femhot_pcg in FP64 mode plus the solver state, each piece
-// 256-byte aligned.
-static size_t pcg_async_ws_bytes(const Ctx *c, bool node_blocked) {
-  if (node_blocked) {
-    const TilePlan tp = tile_plan<double>(c);
-    if (tp.ok) return 6 * r256(sizeof(double) * c->Ndof) + r256(sizeof(double) * 8 * tp.G) + r256(sizeof(PcgState));
-  }
-  const size_t vec64 = sizeof(double) * c->Ndof;
-  const size_t nsp = spmv_plan(c->Ndof, c->nnz, c->ndpn, node_blocked).blocks;
-  return r256(3 * NBR * sizeof(double)) + r256(NBR * sizeof(double)) + r256(nsp * sizeof(double)) +
-         r256(8 * sizeof(double)) + 5 * r256(vec64) + r256(sizeof(PcgState));
-}
-
 static int pcg_async_core(Ctx *c, bool node_blocked, const long long *row_ptr, const int *col_idx,
                           const double *vals, const double *b, double *x, double tol, int iterations,
                           const int *outer, const PcgState **state_out, int *iters, double *rel_res, int *status,
@@ -854,7 +857,7 @@ static int pcg_async_core(Ctx *c, bool node_blocked, const long long *row_ptr, c
   const size_t vec64 = sizeof(double) * n;
   const SpmvPlan sp = spmv_plan(n, nnz, c->ndpn, node_blocked);
   const size_t nsp = sp.blocks;
-  const size_t need = pcg_async_ws_bytes(c, node_blocked);
+  const size_t need = pcg_ws_bytes(c);
   if (c->ws_bytes < need) {  // sized once; never inside a graph capture
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     FH_HIP(hipStreamIsCapturing(s, &cs));
@@ -1158,7 +1161,7 @@ extern "C" int femhot_newton_async(femhot_ctx *h, const double *field, double *u
   const size_t need = up(sizeof(double) * std::max<long long>(c->nnz, 1)) + 4 * up(sizeof(double) * n) +
                       up(sizeof(double) * NBR) + up(sizeof(NewtonState));
   if (!c->have_pattern || c->newton_ws.bytes < need || !c->newton_dval_ready ||
-      c->ws_bytes < pcg_async_ws_bytes(c, true)) {
+      c->ws_bytes < pcg_ws_bytes(c)) {
     FH_CHECK_ARG(!capturing, FEMHOT_ERR_ARG,
                  "femhot_newton_async: make one uncaptured call on this context first (it builds the pattern and sizes "
                  "the workspaces), so captured calls allocate nothing");
@@ -1175,7 +1178,7 @@ extern "C" int femhot_newton_async(femhot_ctx *h, const double *field, double *u
       FH_HIP(hipMalloc(&c->newton_ws.ptr, need_now));
       c->newton_ws.bytes = need_now;
     }
-    if ((rc = ensure_workspace(c, pcg_async_ws_bytes(c, true)))) return rc;
+    if ((rc = ensure_workspace(c, pcg_ws_bytes(c)))) return rc;
   }
   char *ws = (char *)c->newton_ws.ptr;
   auto take = [&](size_t bytes) {

@@ -242,7 +242,9 @@ int femhot_pcg(femhot_ctx *ctx, int mode, const long long *row_ptr, const int *c
  * iterations' kernels return at once.  iters (int), rel_res (double) and status (int: 1 converged,
  * 2 non-finite residual, 3 iterations spent) are DEVICE pointers (any may be NULL), written at the end
  * of the stream's work.  Allocates nothing once the context's solver workspace is sized (its first
- * uncaptured call, or a femhot_pcg call), so a whole solve can be captured into a HIP graph.  mode:
+ * uncaptured call, or a femhot_pcg call), so a whole solve can be captured into a HIP graph; later FP64
+ * solves on the context leave the workspace where it is (the first femhot_pcg in FEMHOT_F32 mode needs a
+ * larger one: make it before capturing).  mode:
  * FEMHOT_F64 (| FEMHOT_PCG_CONTEXT_PATTERN); the context's pattern must be built.  No counterpart in the
  * reference, whose iterative solve returns to the host (fe_solver.py:60-78); for callers that capture
  * solves or keep the host out of the loop. */
