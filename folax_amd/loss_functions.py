@@ -301,14 +301,14 @@ class _BatchLoss(torch.autograd.Function):
         ctx.loss = loss
         ctx.body = need_u and loss.physics == L.NEOHOOKE and loss._has_body_force()
         keep_p = ctx.body or (need_p and loss.physics != L.MECHANICAL)
-        ctx.save_for_backward(params if keep_p else None, full if keep_p else None, R, en, low, high)
+        ctx.save_for_backward(params if keep_p else None, full if keep_p else None, R, en)
         ctx.shape, ctx.dtype = params.shape, dofs.dtype
         return mean, low, high
 
     @staticmethod
     def backward(ctx, g, g_low, g_high):
         loss = ctx.loss
-        params, full, R, en, low, high = ctx.saved_tensors
+        params, full, R, en = ctx.saved_tensors
         flags, batch = loss._flags(), en.shape[0]
         plain = g_low is None and g_high is None and not torch.is_grad_enabled()
         if plain and g is not None:
@@ -316,9 +316,10 @@ class _BatchLoss(torch.autograd.Function):
         if not plain:  # each sample's weight: 1 / B of the mean's gradient, the extremes' shared by their ties
             e = en.sum(dim=1).to(ctx.dtype)
             s = torch.zeros_like(e) if g is None else (g / batch).expand(batch)
-            for ge, at in ((g_low, low), (g_high, high)):
-                if ge is not None:
-                    tie = (e == at).to(e.dtype)
+            for ge, extreme in ((g_low, torch.amin), (g_high, torch.amax)):
+                if ge is not None:  # the extreme of e itself: the kernel adds a sample's segments in another order
+                    at = extreme(e)
+                    tie = ((e == at) | (e.isnan() & at.isnan())).to(e.dtype)
                     s = s + ge * tie / tie.sum()
             s = s.reshape(-1, 1)
         elif g is None:
