@@ -45,6 +45,16 @@ def _as_device_tensor(x, dtype=None, device=None):
     return torch.as_tensor(np.asarray(x), dtype=dtype or torch.float64, device=device).contiguous()
 
 
+def _has_memory(t):
+    """Whether a kernel can read t: the tensors of a batched gradient (is_grads_batched) stand for several and
+    have no memory of their own."""
+    try:
+        t.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 class FiniteElementLoss:
     """Base FE loss (fe_loss.py:19-318)."""
 
@@ -310,7 +320,8 @@ class _BatchLoss(torch.autograd.Function):
         loss = ctx.loss
         params, full, R, en = ctx.saved_tensors
         flags, batch = loss._flags(), en.shape[0]
-        plain = g_low is None and g_high is None and not torch.is_grad_enabled()
+        plain = (g_low is None and g_high is None and not torch.is_grad_enabled()
+                 and (g is None or _has_memory(g)))
         if plain and g is not None:
             g = g.contiguous()
         if not plain:  # each sample's weight: 1 / B of the mean's gradient, the extremes' shared by their ties
@@ -365,7 +376,7 @@ class _BatchResidualNorm(torch.autograd.Function):
         flags = loss._flags() | L.MASK_DIRICHLET | (L.PICARD if ctx.picard else 0)
         loss._tune(L.OP_VJP, params, full, R)
         need_p, need_u = ctx.needs_input_grad[1:3]
-        if torch.is_grad_enabled():  # create_graph: the factor stays in the graph
+        if torch.is_grad_enabled() or not _has_memory(g):  # create_graph: the factor stays in the graph
             gu, gd = loss.ctx.residual_vjp(params, full, R, want_gu=need_u, want_gd=need_p, flags=flags)
             return None, gd * g if need_p else None, gu * g if need_u else None, None
         gu, gd = loss.ctx.residual_vjp(params, full, R, want_gu=need_u, want_gd=need_p, flags=flags,
