@@ -8,7 +8,7 @@ and U[c] = N.u_c at each Gauss point, fe_response.py:61-66, 92-113).
 What runs where:
 * the Gauss-point geometry (w detJ, N, dN/dx) comes from the library (femhot_gauss_point_data);
 * the nodal field and state are brought to the Gauss points, and Gauss-point terms back to the nodes,
-  by the library's gather kernels;
+  by the library's gather kernels (under torch's transforms and traces, by torch's own operators);
 * phi is evaluated on the device with torch on all Gauss points at once, and its derivatives with
   respect to the Gauss-point field and state come from torch autograd of that evaluation (the
   formula is arbitrary Python, as the reference's jax.grad of its eval'd lambda);
@@ -19,9 +19,10 @@ What runs where:
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib as L
-from .loss_functions import FiniteElementLoss, _as_device_tensor
+from .loss_functions import FiniteElementLoss, _as_device_tensor, _has_memory
 
 
 class _ArrayNamespace:
@@ -37,38 +38,61 @@ class _ArrayNamespace:
         return getattr(torch, name)
 
 
+def _kernels_read(*tensors):
+    """Whether the gather kernels can take these tensors: plain ones with memory of their own, outside torch's
+    transforms (functorch, forward mode, batched gradients) and traces, which need operators they know."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter)
+                and not torch._C._functorch.is_functorch_wrapped_tensor(t) and _has_memory(t) for t in tensors)
+            and forward_ad._current_level < 0 and not torch._C._len_torch_dispatch_stack()
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
+def _point_values(r, d, u):
+    """N.d (n_elems, G) and N.u (dofs per node, n_elems, G) of response r's mesh: by the kernel, or by torch's own
+    operators where that cannot be (the linear map is the same)."""
+    if _kernels_read(d, u):
+        return _PointValues.apply(r, d, u)
+    N, conn = r._geometry(u.dtype, u.device)[0], r._connectivity(u.device)
+    return d[conn] @ N.T, u.view(-1, r.fe_loss.number_dofs_per_node)[conn].permute(2, 0, 1) @ N.T
+
+
+def _point_gather(r, q):
+    """The transpose of _point_values per component: q (ncomp, n_elems, G) -> (n_nodes, ncomp)."""
+    if _kernels_read(q):
+        return _PointGather.apply(r, q)
+    N, conn = r._geometry(q.dtype, q.device)[0], r._connectivity(q.device)
+    corners = (q @ N).permute(1, 2, 0).reshape(-1, q.shape[0])
+    zero = torch.zeros(r.fe_loss.ctx.n_nodes, q.shape[0], dtype=q.dtype, device=q.device)
+    return zero.index_add(0, conn.reshape(-1), corners)
+
+
 class _PointValues(torch.autograd.Function):
     """N.d and N.u at the Gauss points; its transpose is the gather of _PointGather, so both differentiate
     to any order."""
 
     @staticmethod
-    def forward(ctx, loss, d, u):
-        ctx.loss, ctx.n, ctx.shapes = loss, d.numel(), (d.shape, u.shape)
-        return loss.ctx.gauss_point_values(d.contiguous(), u.contiguous(), loss.num_gp)
+    def forward(ctx, r, d, u):
+        ctx.r, ctx.shapes = r, (d.shape, u.shape)
+        return r.fe_loss.ctx.gauss_point_values(d.contiguous(), u.contiguous(), r.fe_loss.num_gp)
 
     @staticmethod
     def backward(ctx, gd, gu):
-        d = _PointGather.apply(ctx.loss, gd.unsqueeze(0)).reshape(-1) if ctx.needs_input_grad[1] else None
-        if d is not None and ctx.n != d.numel():
-            d = torch.nn.functional.pad(d, (0, ctx.n - d.numel()))
-        return (None, d.reshape(ctx.shapes[0]) if d is not None else None,
-                _PointGather.apply(ctx.loss, gu).reshape(ctx.shapes[1]) if ctx.needs_input_grad[2] else None)
+        return (None, _point_gather(ctx.r, gd.unsqueeze(0)).reshape(ctx.shapes[0]) if ctx.needs_input_grad[1] else None,
+                _point_gather(ctx.r, gu).reshape(ctx.shapes[1]) if ctx.needs_input_grad[2] else None)
 
 
 class _PointGather(torch.autograd.Function):
     """sum of N_a q at the nodes, (n_nodes, ncomp); the transpose of _PointValues per component."""
 
     @staticmethod
-    def forward(ctx, loss, q):
-        ctx.loss, ctx.ncomp = loss, q.shape[0]
-        return loss.ctx.gauss_point_gather(q, loss.num_gp)
+    def forward(ctx, r, q):
+        ctx.r, ctx.ncomp = r, q.shape[0]
+        return r.fe_loss.ctx.gauss_point_gather(q, r.fe_loss.num_gp)
 
     @staticmethod
     def backward(ctx, g):
-        loss = ctx.loss
-        zero = torch.zeros(loss.ctx.n_dofs, dtype=g.dtype, device=g.device)
-        parts = [_PointValues.apply(loss, g[:, c].contiguous(), zero)[0] for c in range(ctx.ncomp)]
-        return None, torch.stack(parts)
+        zero = torch.zeros(ctx.r.fe_loss.ctx.n_dofs, dtype=g.dtype, device=g.device)
+        return None, torch.stack([_point_values(ctx.r, g[:, c].contiguous(), zero)[0] for c in range(ctx.ncomp)])
 
 
 class FiniteElementResponse:
@@ -94,6 +118,7 @@ class FiniteElementResponse:
         self.response_function = eval(f"lambda {', '.join(variables)}: {self.response_formula}",
                                       {"jnp": _ArrayNamespace()})
         self._gp = {}
+        self._conn = None
         self._has_both = False
         self.fe_loss.ctx.build_incidence()
         self.initialized = True
@@ -105,6 +130,13 @@ class FiniteElementResponse:
             self._gp[key] = self.fe_loss.ctx.gauss_point_data(self.fe_loss.num_gp, dtype=dtype, device=device)
         return self._gp[key]
 
+    def _connectivity(self, device):
+        if self._conn is None or self._conn.device != device:
+            with torch._C._DisableFuncTorch():  # kept beyond the transform that first needs it
+                self._conn = torch.as_tensor(self.fe_loss.fe_mesh.GetElementsNodes(self.fe_loss.element_type),
+                                             dtype=torch.int64, device=device)
+        return self._conn
+
     def _inputs(self, control, dofs):
         u = _as_device_tensor(dofs)
         d = _as_device_tensor(control, dtype=u.dtype, device=u.device)
@@ -113,7 +145,12 @@ class FiniteElementResponse:
     def _integrand(self, d, u):
         """w detJ (Ne, G) and, at the Gauss points, N.d (Ne, G) and N.u (ndpn, Ne, G): U[c] is component c."""
         _, wdet, _ = self._geometry(u.dtype, u.device)
-        gp_d, gp_u = _PointValues.apply(self.fe_loss, d, u)
+        n, p = self.fe_loss.ctx.n_nodes, self.fe_loss.number_dofs_per_node
+        if d.numel() < n or u.numel() < n * p:
+            raise IndexError(f"a response reads {n} nodal control values and {n * p} dofs")
+        if d.numel() > n or u.numel() > n * p:  # the nodes' values come first
+            d, u = d[:n], u.view(-1, p)[:n].reshape(-1)
+        gp_d, gp_u = _point_values(self, d, u)
         return wdet, gp_d, gp_u
 
     # ---- reference API ----
@@ -173,8 +210,7 @@ class FiniteElementResponse:
             ge = torch.einsum("eg,egaj->eaj", wphi, dndx)                # (Ne, n, dim)
             if ge.shape[-1] < 3:
                 ge = torch.nn.functional.pad(ge, (0, 3 - ge.shape[-1]))
-            conn = torch.as_tensor(self.fe_loss.fe_mesh.GetElementsNodes(self.fe_loss.element_type),
-                                   dtype=torch.int64, device=u.device)
+            conn = self._connectivity(u.device)
             dfdX = torch.zeros(self.fe_loss.fe_mesh.GetNumberOfNodes(), 3, dtype=u.dtype, device=u.device)
             dfdX.index_add_(0, conn.reshape(-1), ge.reshape(-1, 3))
             return dfdX.reshape(-1) + self.fe_loss.ComputeResidualShapeVJP(d, u, lam)
