@@ -194,9 +194,8 @@ static size_t lds_limit() {
 // must already be built, nothing is allocated and no timing events are recorded.
 static int run_chunk_cfg(Ctx *c, int dtype, int mode, int batch, const void *field, long long fs, const void *u,
                          long long us, const void *w, long long ws, void *ou, long long ous, void *od, long long ods,
-                         double *energy, unsigned flags, hipStream_t s, ChunkConfig cfg,
+                         double *energy, unsigned flags, hipStream_t s, const ChunkConfig &cfg,
                          void *fixed_ws = nullptr, size_t fixed_bytes = 0, const void *wscale = nullptr) {
-  if (wscale) cfg.dma = false;  // the LDS-DMA kernel brings the cotangent to LDS as it is
   const ChunkPlan *plan = nullptr;
   int rc;
   if (fixed_ws) {

@@ -210,6 +210,8 @@ __global__ __launch_bounds__(BLOCK) void k_chunk_pipe(ChunkArgs A) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_items = A.n_chunks * A.n_sblocks;
+  // (the cotangent streams to LDS as it is and is scaled on its way to the element)
+  const R wsc = MODE == MODE_VJP && A.wscale ? *reinterpret_cast<const R *>(A.wscale) : R(1);
   if ((int)blockIdx.x >= n_items) return;  // uniform over the workgroup
   __shared__ __align__(16) int geo[4];     // chunk offsets of the step after next (DMA)
   PipeStep S = first_step(A, blockIdx.x);
@@ -280,7 +282,7 @@ __global__ __launch_bounds__(BLOCK) void k_chunk_pipe(ChunkArgs A) {
 #pragma unroll
         for (int a = 0; a < N; ++a)
 #pragma unroll
-          for (int c = 0; c < P; ++c) w[a * P + c] = W[c * cap64 + l[a]];
+          for (int c = 0; c < P; ++c) w[a * P + c] = wsc * W[c * cap64 + l[a]];
         elem_vjp<R, ET, PH, NGP>(el, w, A.pp, picard, ro, gd);
       } else {
         R pi;
