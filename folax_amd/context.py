@@ -49,6 +49,7 @@ class FemhotContext:
         self.elem_type = elem_type
         self.et = L.ELEMENT_TYPES[elem_type]
         self.physics = physics
+        self.num_gp = int(num_gp) or (1 if self.et == L.TET4 else 2)
         self.n_nodes = coords.shape[0]
         self.n_elems = conn.shape[0]
         didx = np.ascontiguousarray(np.zeros(0) if dirichlet_idx is None else dirichlet_idx, dtype=np.int64)
@@ -252,13 +253,20 @@ class FemhotContext:
         self._check_in(field.view(1, -1), "field", self._field_size(flags), 1, dt, dev)
         gx = torch.empty(self.n_nodes, 3, dtype=dt, device=dev)
         dim = 2 if self.et == L.QUAD4 else 3
-        if wphi is not None and (wphi.dtype != dt or wphi.device != dev or not wphi.is_contiguous()
-                                 or wphi.numel() % self.n_elems):
-            raise ValueError("wphi must be a contiguous (n_elems, G) tensor of u's dtype and device")
+        if wphi is not None:
+            G = self._points(self.num_gp)
+            if wphi.dtype != dt or wphi.device != dev or not wphi.is_contiguous() or wphi.numel() != self.n_elems * G:
+                raise ValueError(f"wphi must be a contiguous ({self.n_elems}, {G}) tensor of u's dtype and device")
         scratch = torch.empty(self.n_elems * self.nodes_per_elem * dim, dtype=dt, device=dev)
         L.check(self._lib.femhot_shape_gradient(self._h, _dtype_code(u), _ptr(field), _ptr(u), _ptr(w), _ptr(wphi),
                                                 _ptr(scratch), _ptr(gx), flags, _stream()))
         return gx
+
+    def _points(self, num_gp):
+        """Gauss points per element; num_gp must be the context's rule, which the kernels use."""
+        if num_gp != self.num_gp:
+            raise ValueError(f"the context integrates with Gauss rule {self.num_gp}, not {num_gp}")
+        return L.gauss_points_per_element(self.et, num_gp)
 
     def build_incidence(self):
         """The node incidence that gauss_point_gather walks (built by its first call otherwise, not in a
@@ -267,12 +275,14 @@ class FemhotContext:
 
     def gauss_point_values(self, field, u, num_gp):
         """N.d (n_elems, G) and N.u (dofs_per_node, n_elems, G) of a nodal field and a solution."""
-        G = L.gauss_points_per_element(self.et, num_gp)
+        G = self._points(num_gp)
         gd = torch.empty(self.n_elems, G, dtype=u.dtype, device=u.device)
         gu = torch.empty(self.dofs_per_node, self.n_elems, G, dtype=u.dtype, device=u.device)
         self._check_in(u.view(1, -1), "u", self.n_dofs, 1, u.dtype, u.device)
-        if field.dtype != u.dtype or field.device != u.device or field.numel() < self.n_nodes:
-            raise IndexError(f"field must hold {self.n_nodes} nodal values of u's dtype and device")
+        if field.dtype != u.dtype or field.device != u.device or not field.is_contiguous():
+            raise ValueError("field must be a contiguous tensor of u's dtype and device")
+        if field.numel() < self.n_nodes:
+            raise IndexError(f"field must hold {self.n_nodes} nodal values")
         L.check(self._lib.femhot_gauss_point_values(self._h, _dtype_code(u), _ptr(field), _ptr(u), _ptr(gd), _ptr(gu),
                                                     _stream()))
         return gd, gu
@@ -280,8 +290,10 @@ class FemhotContext:
     def gauss_point_gather(self, q, num_gp, out=None):
         """sum over elements and Gauss points of N_a q at the nodes: q (ncomp, n_elems, G) -> (n_nodes, ncomp);
         out: a contiguous tensor of that shape to add into."""
-        G = L.gauss_points_per_element(self.et, num_gp)
+        G = self._points(num_gp)
         q = q.contiguous()
+        if not q.is_cuda:
+            raise ValueError("q must be a device tensor")
         if q.dim() != 3 or tuple(q.shape[1:]) != (self.n_elems, G):
             raise ValueError(f"q must have shape (ncomp, {self.n_elems}, {G})")
         flags = 0 if out is None else L.ACCUMULATE
