@@ -111,7 +111,7 @@ class FiniteElementLoss:
         # point-data heterogeneity field when material_dict names one, as
         # mechanical_saint_venant.py:59-66 does)
         self.parametric_boundary_learning = bool(self.loss_settings.get("parametric_boundary_learning"))
-        self.get_param_function = lambda x: x
+        self.get_param_function = self._given_params
         md = self.loss_settings.get("material_dict", {})
         if self.parametric_boundary_learning and "heterogeneity_field_name" in md:
             name = md["heterogeneity_field_name"]
@@ -135,6 +135,7 @@ class FiniteElementLoss:
                                  self.fe_mesh.GetElementsNodes(self.element_type), num_gp=num_gp,
                                  dirichlet_idx=self.dirichlet_indices, dirichlet_val=self.dirichlet_values,
                                  segment_offsets=self.loss_settings.get("segment_offsets"), **self._material())
+        self._ctx_dirichlet = self.dirichlet_indices.copy(), self.dirichlet_values.copy()
         self._dir_idx_t = None
         self.initialized = True
 
@@ -148,11 +149,20 @@ class FiniteElementLoss:
             self._tuned.add(key)
 
     def _one_call(self, bp, bd):
-        """Whether a batch loss runs through its one-call entry points: device tensors of one floating type,
-        fixed Dirichlet values."""
-        return (not self.parametric_boundary_learning and isinstance(bp, torch.Tensor) and isinstance(bd, torch.Tensor)
+        """Whether a batch loss runs through its one-call entry points: device tensors of one floating type, the
+        base class's dof and parameter vectors, and the Dirichlet values that the context holds."""
+        if not (not self.parametric_boundary_learning and isinstance(bp, torch.Tensor) and isinstance(bd, torch.Tensor)
                 and bd.is_cuda and bp.device == bd.device and bp.dtype == bd.dtype
-                and bd.dtype in (torch.float32, torch.float64) and bp.dim() == 2 and bd.dim() == 2)
+                and bd.dtype in (torch.float32, torch.float64) and bp.dim() == 2 and bd.dim() == 2):
+            return False
+        base = FiniteElementLoss
+        for name in ("GetFullDofVector", "GetParametersVectors"):  # a subclass's (or an object's) own
+            if getattr(getattr(self, name), "__func__", None) is not getattr(base, name):
+                return False
+        if self.get_param_function is not base._given_params:
+            return False
+        self._dir_idx(bd.device)
+        return self._dir_in_ctx
 
     def _has_body_force(self):
         return bool(np.any(np.asarray(self.loss_settings.get("body_foce", [0.0]), dtype=np.float64) != 0.0))
@@ -165,6 +175,9 @@ class FiniteElementLoss:
         if self._dir_idx_t is None or self._dir_idx_t.device != device:
             self._dir_idx_t = torch.as_tensor(self.dirichlet_indices, dtype=torch.int64, device=device)
             self._dir_val_t = torch.as_tensor(self.dirichlet_values, dtype=torch.float64, device=device)
+            idx, val = self._ctx_dirichlet
+            self._dir_in_ctx = (np.array_equal(self.dirichlet_indices, idx)
+                                and np.array_equal(self.dirichlet_values, val, equal_nan=True))
         return self._dir_idx_t, self._dir_val_t
 
     def Finalize(self):
@@ -192,6 +205,10 @@ class FiniteElementLoss:
         else:
             out[..., idx] = val.to(u.dtype)
         return out
+
+    @staticmethod
+    def _given_params(param_vector):
+        return param_vector
 
     def _heterogeneity_params(self, param_vector):
         p = torch.as_tensor(self.heterogeneity_field, device=param_vector.device, dtype=param_vector.dtype)

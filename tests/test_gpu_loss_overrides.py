@@ -1,0 +1,69 @@
+"""Batch losses with a subclass's dof or parameter vectors, an object's own, or Dirichlet values set after
+initialization: the loss is that of the vectors it was told to use."""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _losses():
+    from folax_amd import loss_functions as lf
+
+    class Doubled(lf.ThermalLoss2DQuad):
+        def GetParametersVectors(self, param_vector):
+            return 2.0 * super().GetParametersVectors(param_vector)
+
+    class Shifted(lf.ThermalLoss2DQuad):
+        def GetFullDofVector(self, known_dofs, unknown_dofs):
+            return super().GetFullDofVector(known_dofs, unknown_dofs) + 0.25
+
+    return lf.ThermalLoss2DQuad, Doubled, Shifted
+
+
+def _make(cls):
+    from folax_amd.mesh import create_2D_square_mesh
+    loss = cls("l", {"dirichlet_bc_dict": {"T": {"left": 1.0, "right": 0.0}}, "beta": 0.5, "c": 2},
+               create_2D_square_mesh(1.0, 8))
+    loss.Initialize()
+    return loss
+
+
+@pytest.mark.parametrize("how", ["subclass parameters", "subclass dofs", "object parameters", "object dofs",
+                                 "parameter function", "values", "values in place"])
+def test_vectors_in_use(how):
+    base, doubled, shifted = _losses()
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    f, u = (torch.rand(3, 64, generator=gen, device="cuda", dtype=torch.float64) + 0.5 for _ in range(2))
+    plain = _make(base)
+    left = plain.fe_mesh.GetNodeSet("left")
+    loss = _make({"subclass parameters": doubled, "subclass dofs": shifted}.get(how, base))
+    field = f
+    full = plain.GetFullDofVector(f, u)
+    if how in ("subclass parameters", "object parameters", "parameter function"):
+        field = 2.0 * f
+        if how == "object parameters":
+            loss.GetParametersVectors = lambda p: 2.0 * p
+        elif how == "parameter function":
+            loss.get_param_function = lambda p: 2.0 * p
+    elif how in ("subclass dofs", "object dofs"):
+        full = full + 0.25
+        if how == "object dofs":
+            loss.GetFullDofVector = lambda known, dofs: plain.GetFullDofVector(known, dofs) + 0.25
+    else:
+        full = full.clone()
+        full[:, torch.as_tensor(left, device="cuda")] = 3.0
+        if how == "values":
+            loss.dirichlet_values = 3.0 * loss.dirichlet_values
+        else:
+            loss.dirichlet_values *= 3.0
+    energy = sum(plain.ComputeTotalEnergy(field[b], full[b]) for b in range(3)) / 3
+    norm = sum(0.5 * (plain.ComputeResidual(field[b], full[b]) ** 2).sum() for b in range(3))
+    for call, want in ((lambda p: loss.ComputeBatchLoss(p, u)[0], energy),
+                       (lambda p: loss.ComputeBatchResidualNormLoss(p, u), norm)):
+        p = f.clone().requires_grad_(True)
+        value = call(p)
+        assert abs(float(value) - float(want)) <= 1e-13 * abs(float(want))  # sums of 64 nodes
+        # both are homogeneous in the conductivity, of degree 1 and 2
+        degree = 2.0 if want is norm else 1.0
+        (g,) = torch.autograd.grad(value, p)
+        assert abs(float((g * f).sum()) - degree * float(want)) <= 1e-12 * degree * abs(float(want))
