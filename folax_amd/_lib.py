@@ -40,7 +40,7 @@ EXPORTED = [
     "femhot_gauss_point_data", "femhot_energy_grad_noalloc", "femhot_pcg_async", "femhot_newton_async",
     "femhot_chunk_plan_check", "femhot_residual_vjp_scaled", "femhot_batch_residual_norm", "femhot_batch_loss",
     "femhot_scale", "femhot_shape_gradient", "femhot_gauss_point_values", "femhot_gauss_point_gather",
-    "femhot_incidence",
+    "femhot_incidence", "femhot_pcg_wait_limit",
 ]
 
 OP_RESIDUAL, OP_VJP, OP_ENERGY_GRAD, OP_TANGENT = 0, 1, 2, 3
@@ -110,6 +110,7 @@ def lib():
     L.femhot_batch_loss.argtypes = [vp, i32, i32, vp, ll, vp, ll, vp, vp, vp, vp, vp, vp, u32, vp]
     L.femhot_shape_gradient.argtypes = [vp, i32, vp, vp, vp, vp, vp, vp, u32, vp]
     L.femhot_incidence.argtypes = [vp]
+    L.femhot_pcg_wait_limit.argtypes = [vp, i32]
     L.femhot_gauss_point_values.argtypes = [vp, i32, vp, vp, vp, vp, vp]
     L.femhot_gauss_point_gather.argtypes = [vp, i32, i32, vp, vp, u32, vp]
     L.femhot_scale.argtypes = [i32, ll, vp, vp, dbl, vp, vp]

@@ -129,6 +129,10 @@ struct Ctx {
   size_t ws_bytes = 0;
   void *d_ws = nullptr;
   double *h_pinned = nullptr;  // pinned host scratch (1024 doubles: the solver's reduction partials)
+  // one-launch solves: looks at a value that another workgroup publishes before a wait gives up (seconds),
+  // and whether one has given up during the current call (its further linear solves then do not try again)
+  int tile_looks = 1 << 21;
+  bool tile_gave_up = false;
 };
 
 int ensure_pattern(Ctx *c);

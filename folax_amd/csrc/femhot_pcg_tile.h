@@ -16,8 +16,9 @@
 // fence and no second message.  Slots alternate by the iteration's parity; an owner resets a slot after
 // every reader has consumed it (it has passed the next exchange) and waits for that store before it
 // publishes to the exchange that precedes the slot's reuse.  Polls are bounded: a workgroup that waits
-// too long raises `fail`, leaves, and the caller solves with the launched kernels (x is written only at
-// the end of a solve).
+// too long raises `fail` and leaves, after which every other one's waits end too, and the caller solves with the
+// launched kernels.  A workgroup may give up just as the others converge and store their parts of x, so the
+// start vector is kept (x0) and put back first.
 //
 // p of a neighbour is formed by its readers as z + beta p (as by its owner: one FMA, the same bits), so
 // the exchange that sums r.z also carries the vector the SpMV needs.
@@ -29,7 +30,6 @@ namespace femhot {
 constexpr int TILE_U = 4;       // neighbour blocks per lane
 constexpr int TILE_T = 512;     // threads per workgroup
 constexpr int TILE_RANGE = 65536;  // most node ids between the first and last column of a workgroup's rows
-constexpr int TILE_SPIN = 1 << 21;
 
 // Solver state shared by the forms: status 0 running, 1 converged, 2 non-finite residual, 3 iteration
 // budget spent, 4 skipped (an enclosing solve has ended).
@@ -48,6 +48,7 @@ struct TileArgs {
   const int *doff;  // offset of each row's diagonal within the row, -1 for an empty row
   const double *b;
   void *x;          // initial guess in, solution out (T)
+  void *x0;         // the initial guess, kept by k_tile_clear (T)
   void *z[2];       // published z by parity (n, T)
   double *pa;       // (2 parities, 3, G): r.z, r.r, b.b
   double *pc;       // (2 parities, G): p.Ap
@@ -55,6 +56,7 @@ struct TileArgs {
   double bnorm;     // < 0: the solve takes ||b|| itself
   double tol;
   int maxiter, check;
+  int looks;        // before a wait gives up
   PcgState *st;
   int *fail;
 };
@@ -76,11 +78,13 @@ template <class T> __device__ __forceinline__ typename TileBits<T>::U tile_peek(
   using U = typename TileBits<T>::U;
   return __hip_atomic_load(reinterpret_cast<const U *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The value published at p; `seen` may hold an earlier look at it.  Ends after TILE_SPIN looks.
-template <class T> __device__ __forceinline__ T tile_wait(const T *p, typename TileBits<T>::U seen, int &bad) {
+// The value published at p; `seen` may hold an earlier look at it.  Gives up (bad) after `looks` looks, and at
+// once where this lane has given up before.
+template <class T>
+__device__ __forceinline__ T tile_wait(const T *p, typename TileBits<T>::U seen, int looks, int &bad) {
   using U = typename TileBits<T>::U;
   for (int n = 0; seen == ~U(0); ++n) {
-    if (n >= TILE_SPIN) {
+    if (bad || n >= looks) {
       bad = 1;
       return T(0);
     }
@@ -353,9 +357,9 @@ __global__ __launch_bounds__(TILE_T) void k_pcg_resident(TileArgs A) {
 #pragma unroll
       for (int j = 0; j < ZN; ++j) seen[j] = tile_peek<T>(zk + zo[j]);
       if (tid < G) {
-        pz = tile_wait<double>(pa + tid, s0, bad);
-        pr = tile_wait<double>(pa + G + tid, s1, bad);
-        if (k == 0) pb = tile_wait<double>(pa + 2 * G + tid, ~0ull, bad);
+        pz = tile_wait<double>(pa + tid, s0, A.looks, bad);
+        pr = tile_wait<double>(pa + G + tid, s1, A.looks, bad);
+        if (k == 0) pb = tile_wait<double>(pa + 2 * G + tid, ~0ull, A.looks, bad);
       }
       if (bad) bad_s = 1;
       if (k == 0) tbb = tile_block_sum(pb, red[2]);
@@ -394,7 +398,7 @@ __global__ __launch_bounds__(TILE_T) void k_pcg_resident(TileArgs A) {
 #pragma unroll
       for (int j = 0; j < ZN; ++j) {
         const int i = tid + j * TILE_T;
-        if (i < nh) pl[i] = tile_axpy<T>(beta, pl[i], tile_wait<T>(zk + zo[j], seen[j], bad));
+        if (i < nh) pl[i] = tile_axpy<T>(beta, pl[i], tile_wait<T>(zk + zo[j], seen[j], A.looks, bad));
       }
       for (int i0 = tid + ZN * TILE_T; i0 < nh; i0 += ZN * TILE_T) {
         const T *zr[ZN];
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(TILE_T) void k_pcg_resident(TileArgs A) {
 #pragma unroll
         for (int j = 0; j < ZN; ++j) {
           const int i = i0 + j * TILE_T;
-          if (i < nh) pl[i] = tile_axpy<T>(beta, pl[i], tile_wait<T>(zr[j], seen[j], bad));
+          if (i < nh) pl[i] = tile_axpy<T>(beta, pl[i], tile_wait<T>(zr[j], seen[j], A.looks, bad));
         }
       }
     }
@@ -429,7 +433,7 @@ __global__ __launch_bounds__(TILE_T) void k_pcg_resident(TileArgs A) {
       double *pc = A.pc + (size_t)par * G;
       if (tid == 0) tile_publish<double>(pc + wg, tpq);
       double pp = 0.0;
-      if (tid < G) pp = tile_wait<double>(pc + tid, ~0ull, bad);
+      if (tid < G) pp = tile_wait<double>(pc + tid, ~0ull, A.looks, bad);
       if (bad) bad_s = 1;
       tpq = tile_block_sum(pp, red[4]);
       if (bad_s) break;
@@ -464,7 +468,7 @@ __global__ __launch_bounds__(TILE_T) void k_pcg_resident(TileArgs A) {
       tile_reset<double>(po + G + wg);
     }
   }
-  if (status == 0) {  // a wait ran out: x stays as it was
+  if (status == 0) {  // a wait ran out
     if (tid == 0) *A.fail = 1;
     return;
   }
@@ -481,13 +485,14 @@ __global__ __launch_bounds__(TILE_T) void k_pcg_resident(TileArgs A) {
   }
 }
 
-// Slots of the exchanges to the sentinel, the failure flag and the state cleared.
+// Slots of the exchanges to the sentinel, the failure flag and the state cleared, x kept.
 template <class T> __global__ __launch_bounds__(256) void k_tile_clear(TileArgs A, long long n) {
   using U = typename TileBits<T>::U;
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i < n) {
     reinterpret_cast<U *>(A.z[0])[i] = ~U(0);
     reinterpret_cast<U *>(A.z[1])[i] = ~U(0);
+    reinterpret_cast<T *>(A.x0)[i] = reinterpret_cast<const T *>(A.x)[i];
   }
   if (i < 6 * A.G) reinterpret_cast<unsigned long long *>(A.pa)[i] = ~0ull;
   if (i < 2 * A.G) reinterpret_cast<unsigned long long *>(A.pc)[i] = ~0ull;

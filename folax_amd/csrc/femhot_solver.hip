@@ -499,7 +499,7 @@ template <class T> static TilePlan tile_plan(const Ctx *c) {
 
 static size_t r256(size_t b) { return (b + 255) & ~size_t(255); }
 template <class T> static size_t tile_ws_bytes(const Ctx *c, const TilePlan &tp) {
-  return 2 * r256(sizeof(T) * c->Ndof) + r256(sizeof(double) * 8 * tp.G) + 2 * r256(sizeof(PcgState));
+  return 3 * r256(sizeof(T) * c->Ndof) + r256(sizeof(double) * 8 * tp.G) + 2 * r256(sizeof(PcgState));
 }
 
 // Workspace of an FP64 solve on this context, host-checked or enqueued, on the context's pattern or any
@@ -521,7 +521,7 @@ static size_t pcg_ws_bytes(const Ctx *c) {
 }
 
 // One resident solve (k_pcg_resident), synchronised: *st the final state; *ran false when it could not be
-// launched or a wait between its workgroups ran out (x is then untouched).
+// launched or a wait between its workgroups ran out (x is then the initial guess again).
 template <class T>
 static int tile_solve(Ctx *c, const TilePlan &tp, void *ws, const long long *rp, const int *ci, const double *vals,
                       const double *b, T *x, double bnorm, double tol, int maxiter, int check, hipStream_t s,
@@ -542,6 +542,7 @@ static int tile_solve(Ctx *c, const TilePlan &tp, void *ws, const long long *rp,
   A.x = x;
   A.z[0] = take(sizeof(T) * c->Ndof);
   A.z[1] = take(sizeof(T) * c->Ndof);
+  A.x0 = take(sizeof(T) * c->Ndof);
   A.pa = (double *)take(sizeof(double) * 8 * tp.G);
   A.pc = A.pa + 6 * tp.G;
   A.st = (PcgState *)take(sizeof(PcgState));
@@ -554,6 +555,7 @@ static int tile_solve(Ctx *c, const TilePlan &tp, void *ws, const long long *rp,
   A.tol = tol;
   A.maxiter = maxiter;
   A.check = check;
+  A.looks = c->tile_looks;
   const long long nc = std::max<long long>(c->Ndof, 8LL * tp.G);
   hipLaunchKernelGGL((k_tile_clear<T>), dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, A, c->Ndof);
   *ran = false;
@@ -570,7 +572,11 @@ static int tile_solve(Ctx *c, const TilePlan &tp, void *ws, const long long *rp,
     }
     return FEMHOT_OK;
   });
-  if (rc || !*ran) return rc;
+  if (rc) return rc;
+  if (!*ran) {
+    c->tile_gave_up = true;
+    return FEMHOT_OK;
+  }
   struct Out {
     PcgState st;
     int fail;
@@ -580,6 +586,10 @@ static int tile_solve(Ctx *c, const TilePlan &tp, void *ws, const long long *rp,
   FH_HIP(hipStreamSynchronize(s));
   *ran = !o->fail && o->st.status != 0;
   *st = o->st;
+  if (!*ran) {
+    c->tile_gave_up = true;
+    FH_HIP(hipMemcpyAsync(x, A.x0, sizeof(T) * c->Ndof, hipMemcpyDeviceToDevice, s));
+  }
   return FEMHOT_OK;
 }
 
@@ -672,9 +682,10 @@ extern "C" int femhot_spmv(femhot_ctx *h, const long long *row_ptr, const int *c
   return FEMHOT_OK;
 }
 
-extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, const int *col_idx, const double *vals,
-                          const double *b, double *x, double tol, int maxiter, int *iters, double *rel_res,
-                          void *stream) {
+// femhot_pcg, also for the linear solves inside another call (which do not try a one-launch solve again after
+// one has given up).
+static int pcg_call(femhot_ctx *h, int mode, const long long *row_ptr, const int *col_idx, const double *vals,
+                    const double *b, double *x, double tol, int maxiter, int *iters, double *rel_res, void *stream) {
   FH_CHECK_ARG(h && row_ptr && col_idx && vals && b && x, FEMHOT_ERR_ARG, "null argument");
   const bool node_blocked = (mode & FEMHOT_PCG_CONTEXT_PATTERN) != 0;
   mode &= ~FEMHOT_PCG_CONTEXT_PATTERN;
@@ -695,7 +706,7 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
   TilePlan tp;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   FH_HIP(hipStreamIsCapturing(s, &cs));
-  if (node_blocked && cs == hipStreamCaptureStatusNone)
+  if (node_blocked && cs == hipStreamCaptureStatusNone && !c->tile_gave_up)
     tp = mode == FEMHOT_F64 ? tile_plan<double>(c) : tile_plan<float>(c);
   // FP32 mode keeps an FP32 matrix and 5 FP32 vectors, and the resident solve's buffers, beside the FP64 part
   const size_t tile_bytes = mode == FEMHOT_F32 && tp.ok ? tile_ws_bytes<float>(c, tp) : 0;
@@ -803,7 +814,7 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
           if (iters) *iters = it + k_in;
           return FEMHOT_ERR_NONFINITE;
         }
-        if (!ran) tile_ws = nullptr;
+        if (!ran) tile_ws = nullptr;  // the further inner solves do not try again
       }
       if (!ran) cast();
       if (!ran)
@@ -822,6 +833,19 @@ extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, con
     set_error("femhot_pcg: maximum iterations reached");
     return FEMHOT_ERR_NOT_CONVERGED;
   }
+  return FEMHOT_OK;
+}
+
+extern "C" int femhot_pcg(femhot_ctx *h, int mode, const long long *row_ptr, const int *col_idx, const double *vals,
+                          const double *b, double *x, double tol, int maxiter, int *iters, double *rel_res,
+                          void *stream) {
+  if (h) h->c.tile_gave_up = false;
+  return pcg_call(h, mode, row_ptr, col_idx, vals, b, x, tol, maxiter, iters, rel_res, stream);
+}
+
+extern "C" int femhot_pcg_wait_limit(femhot_ctx *h, int looks) {
+  FH_CHECK_ARG(h && looks >= 0, FEMHOT_ERR_ARG, "femhot_pcg_wait_limit: a context and looks >= 0");
+  h->c.tile_looks = looks;
   return FEMHOT_OK;
 }
 
@@ -983,6 +1007,7 @@ extern "C" int femhot_newton(femhot_ctx *h, int mode, const double *field, doubl
                FEMHOT_ERR_ARG,
                "femhot_newton: flags may hold FEMHOT_ELEMENT_FIELD and FEMHOT_SCATTER_{COLOUR,CHUNK,ROWS} only");
   Ctx *c = &h->c;
+  c->tile_gave_up = false;
   int rc = ensure_pattern(c);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
@@ -1038,8 +1063,8 @@ extern "C" int femhot_newton(femhot_ctx *h, int mode, const double *field, doubl
       hipLaunchKernelGGL(k_newton_rhs, grid, dim3(256), 0, s, n, R, b, du);
       int lit = 0;
       double lrel = 0.0;
-      rc = femhot_pcg(h, mode | FEMHOT_PCG_CONTEXT_PATTERN, c->d_row_ptr, c->d_col_idx, vals, b, du, lin_tol,
-                      lin_maxiter, &lit, &lrel, stream);
+      rc = pcg_call(h, mode | FEMHOT_PCG_CONTEXT_PATTERN, c->d_row_ptr, c->d_col_idx, vals, b, du, lin_tol,
+                    lin_maxiter, &lit, &lrel, stream);
       if (rc && rc != FEMHOT_ERR_NOT_CONVERGED) return rc;  // an unconverged solve continues with its iterate
       hipLaunchKernelGGL(k_dot64, dim3(NBR), dim3(256), 0, s, n, du, du, part);
       double dd = 0.0;

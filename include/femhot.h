@@ -237,6 +237,12 @@ int femhot_pcg(femhot_ctx *ctx, int mode, const long long *row_ptr, const int *c
                const double *b, double *x, double rel_tol, int maxiter, int *iters, double *rel_res,
                void *stream);
 
+/* Test hook (no counterpart in the reference): on systems that femhot_pcg solves in one launch, how often a
+ * workgroup looks at a value that another one publishes before it gives up and the call falls back to launched
+ * kernels, from the same initial guess (default 2^21 looks, seconds; 0: it
+ * gives up wherever it would have to wait). */
+int femhot_pcg_wait_limit(femhot_ctx *ctx, int looks);
+
 /* femhot_pcg in FP64 with its convergence test on the device: the host enqueues exactly `iterations`
  * iterations and never waits; once ||r|| <= rel_tol ||b|| (or the residual is not finite) the remaining
  * iterations' kernels return at once.  iters (int), rel_res (double) and status (int: 1 converged,
