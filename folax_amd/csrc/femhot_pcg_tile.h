@@ -8,8 +8,11 @@
 //    four kernels of 2-5 us each whatever the system's size (16-18 us up to 10,000 dofs).  Here the
 //    matrix stays in registers, the search direction of every node the workgroup's rows touch stays in
 //    LDS, and an iteration exchanges only z and the partial dot products: two hops through memory.
-//  * k_tile_init / k_tile_spmv / k_tile_update: one launch per phase, for callers that capture solves
-//    into a graph, where a cooperative launch does not belong.
+//  * k_tile_init / k_tile_spmv (or k_tile_pass, k_tile_dot) / k_tile_update: one launch per phase, for
+//    callers that capture solves into a graph, where a cooperative launch does not belong.  Bound by the
+//    launches: two an iteration and 2-5 us each up to 60,000 dofs.  A captured iteration against the five
+//    kernels of larger systems, which these sizes took before: quads 40 x 40 conduction 15.1 -> 8.9 us,
+//    300 x 300 18.4 -> 15.6, hexahedra 20^3 elastic 18.5 -> 11.4, 45^3 conduction 23.5 -> 21.2.
 //
 // Exchange.  Values are published with agent-scope stores into slots that hold a sentinel (a NaN with all
 // bits set) until then, and read by polling until the sentinel is gone: the value is its own flag, no
@@ -581,20 +584,63 @@ template <int P, int LPN, int S> __global__ __launch_bounds__(TILE_T) void k_til
   }
 }
 
-// Iteration k of parity par: p = z + beta p (p[par] -> p[1 - par]), q = A p, partials of p.q
-template <int P, int LPN, int S>
-__global__ __launch_bounds__(TILE_T) void k_tile_spmv(TileArgs A, TileVecs V, int par, int first) {
-  using G_ = Tile<double, P, LPN, S>;
-  if (A.st->status) return;
-  __shared__ double red[3][TILE_T / 64];
-  const int lane = threadIdx.x % LPN, grp = threadIdx.x / LPN;
-  double beta = 0.0;
-  if (!first) {
-    const double now = tile_sum_slots(A.pa + (size_t)par * 3 * A.G, A.G, red[0]);
-    beta = now / tile_sum_slots(A.pa + (size_t)(1 - par) * 3 * A.G, A.G, red[1]);
+// The test of the enqueued solve, after `it` iterations.
+__device__ __forceinline__ int tile_status(const TileArgs &A, double rr, double bb, int it) {
+  if (!(rr == rr && rr < INFINITY)) return 2;
+  if ((it == 0 && bb == 0.0) || rr <= A.tol * A.tol * bb) return 1;
+  return it >= A.maxiter ? 3 : 0;
+}
+
+// Opens iteration k: every workgroup makes the test that precedes it (workgroup 0 records it; a workgroup that finds
+// its record already there reads the decision it would make) and takes beta.  False: the solve has ended.  A
+// kernel of its own for the test cost 2-3 us an iteration.
+__device__ __forceinline__ bool tile_open(const TileArgs &A, int k, const int *outer, double (*red)[TILE_T / 64],
+                                          double &beta) {
+  if (k > 0 && A.st->status) return false;
+  const int par = k & 1;
+  const double *now = A.pa + (size_t)par * 3 * A.G, *before = A.pa + (size_t)(1 - par) * 3 * A.G;
+  const double rr = tile_sum_slots(now + A.G, A.G, red[0]);
+  const double bb = k == 0 ? tile_sum_slots(now + 2 * A.G, A.G, red[1]) : A.st->bnorm2;
+  const int status = k == 0 && outer && *outer ? 4 : tile_status(A, rr, bb, k);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (k == 0) A.st->bnorm2 = bb;
+    A.st->rr = rr;
+    A.st->iters = k;
+    A.st->status = status;
   }
+  if (status) return false;
+  beta = k == 0 ? 0.0 : tile_sum_slots(now, A.G, red[2]) / tile_sum_slots(before, A.G, red[3]);
+  return true;
+}
+
+// This workgroup's sums of a b and of b b over its dofs, in the order of k_pcg_resident (a thread's S products, then
+// the workgroup's), from LDS, where the dofs are brought by all lanes: LPN - P of LPN lanes own none.
+template <int P, int LPN, int S, bool BOTH>
+__device__ __forceinline__ void tile_products(const TileArgs &A, const double *a, const double *b, double &ab,
+                                              double &bb) {
+  using G_ = Tile<double, P, LPN, S>;
+  const int lane = threadIdx.x % LPN, grp = threadIdx.x / LPN;
+  ab = bb = 0.0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int g = s * G_::NPW + grp;
+    if (lane < P && (long long)blockIdx.x * G_::NPB + g < A.nodes) {
+      ab = __builtin_fma(b[g * P + lane], a[g * P + lane], ab);
+      if (BOTH) bb = __builtin_fma(b[g * P + lane], b[g * P + lane], bb);
+    }
+  }
+}
+
+// Iteration k: p = z + beta p (p[par] -> p[1 - par]), q = A p, partials of p.q
+template <int P, int LPN, int S>
+__global__ __launch_bounds__(TILE_T) void k_tile_spmv(TileArgs A, TileVecs V, int k, const int *outer) {
+  using G_ = Tile<double, P, LPN, S>;
+  __shared__ double red[5][TILE_T / 64];
+  const int lane = threadIdx.x % LPN, grp = threadIdx.x / LPN;
+  double beta;
+  if (!tile_open(A, k, outer, red, beta)) return;
   double q[S], own[S], pq = 0.0;
-  tile_rows<P, LPN, S, false>(A, V, par, beta, q, own);
+  tile_rows<P, LPN, S, false>(A, V, k & 1, beta, q, own);
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const long long node = (long long)blockIdx.x * G_::NPB + s * G_::NPW + grp;
@@ -603,34 +649,74 @@ __global__ __launch_bounds__(TILE_T) void k_tile_spmv(TileArgs A, TileVecs V, in
       pq = __builtin_fma(own[s], q[s], pq);
     }
   }
-  pq = tile_block_sum(pq, red[2]);
+  pq = tile_block_sum(pq, red[4]);
+  if (threadIdx.x == 0) A.pc[blockIdx.x] = pq;
+}
+
+// The same in two kernels: a workgroup per pass, then the partials of p.q.  For many passes of one dof per node
+// (see pcg_async_core).
+template <int P, int LPN>
+__global__ __launch_bounds__(TILE_T) void k_tile_pass(TileArgs A, TileVecs V, int k, const int *outer) {
+  __shared__ double red[4][TILE_T / 64];
+  const int lane = threadIdx.x % LPN, grp = threadIdx.x / LPN;
+  double beta;
+  if (!tile_open(A, k, outer, red, beta)) return;
+  double q[1], own[1];
+  tile_rows<P, LPN, 1, false>(A, V, k & 1, beta, q, own);
+  const long long node = (long long)blockIdx.x * (TILE_T / LPN) + grp;
+  if (lane < P && node < A.nodes) V.q[node * P + lane] = q[0];
+}
+template <int P, int LPN, int S> __global__ __launch_bounds__(TILE_T) void k_tile_dot(TileArgs A, TileVecs V, int par) {
+  constexpr int N = Tile<double, P, LPN, S>::NPB * P;
+  if (A.st->status) return;
+  __shared__ double red[TILE_T / 64], p[N], q[N];
+  const long long r0 = (long long)blockIdx.x * N, n = A.nodes * P;
+#pragma unroll
+  for (int i = threadIdx.x; i < N; i += TILE_T) {
+    p[i] = r0 + i < n ? V.p[1 - par][r0 + i] : 0.0;
+    q[i] = r0 + i < n ? V.q[r0 + i] : 0.0;
+  }
+  __syncthreads();
+  double pq, unused;
+  tile_products<P, LPN, S, false>(A, q, p, pq, unused);
+  pq = tile_block_sum(pq, red);
   if (threadIdx.x == 0) A.pc[blockIdx.x] = pq;
 }
 
 // x += alpha p, r -= alpha q, z, partials of parity 1 - par
 template <int P, int LPN, int S>
 __global__ __launch_bounds__(TILE_T) void k_tile_update(TileArgs A, TileVecs V, int par) {
-  using G_ = Tile<double, P, LPN, S>;
+  constexpr int N = Tile<double, P, LPN, S>::NPB * P, K = (N + TILE_T - 1) / TILE_T;
   if (A.st->status) return;
-  __shared__ double red[4][TILE_T / 64];
-  const int lane = threadIdx.x % LPN, grp = threadIdx.x / LPN;
+  __shared__ double red[4][TILE_T / 64], rl[N], zl[N];
   const double top = tile_sum_slots(A.pa + (size_t)par * 3 * A.G, A.G, red[0]);
   const double alpha = top / tile_sum_slots(A.pc, A.G, red[1]);
-  double *X = reinterpret_cast<double *>(A.x);
-  double rz = 0.0, rr = 0.0;
+  double *X = reinterpret_cast<double *>(A.x), x[K], r[K], z[K];
+  const long long r0 = (long long)blockIdx.x * N, n = A.nodes * P;
 #pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const long long node = (long long)blockIdx.x * G_::NPB + s * G_::NPW + grp;
-    if (lane < P && node < A.nodes) {
-      const long long row = node * P + lane;
-      X[row] = tile_axpy<double>(alpha, V.p[1 - par][row], X[row]);
-      const double r = tile_axpy<double>(-alpha, V.q[row], V.r[row]), z = r * V.dinv[row];
-      V.r[row] = r;
-      V.z[row] = z;
-      rz = __builtin_fma(r, z, rz);
-      rr = __builtin_fma(r, r, rr);
+  for (int j = 0; j < K; ++j) {  // (all loads before the first store, which they might alias)
+    const int i = threadIdx.x + j * TILE_T;
+    const long long row = min(r0 + min(i, N - 1), n - 1);
+    x[j] = tile_axpy<double>(alpha, V.p[1 - par][row], X[row]);
+    r[j] = tile_axpy<double>(-alpha, V.q[row], V.r[row]);
+    z[j] = r[j] * V.dinv[row];
+  }
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const int i = threadIdx.x + j * TILE_T;
+    if (i < N) {
+      rl[i] = r[j];
+      zl[i] = z[j];
+      if (r0 + i < n) {
+        X[r0 + i] = x[j];
+        V.r[r0 + i] = r[j];
+        V.z[r0 + i] = z[j];
+      }
     }
   }
+  __syncthreads();
+  double rz, rr;
+  tile_products<P, LPN, S, true>(A, zl, rl, rz, rr);
   rz = tile_block_sum(rz, red[2]);
   rr = tile_block_sum(rr, red[3]);
   if (threadIdx.x == 0) {
@@ -639,23 +725,15 @@ __global__ __launch_bounds__(TILE_T) void k_tile_update(TileArgs A, TileVecs V, 
   }
 }
 
-// The start of a launched solve, and its test after each iteration (parity: where the new r.r is)
-static __global__ __launch_bounds__(TILE_T) void k_tile_test(TileArgs A, int par, int start, const int *outer) {
-  if (!start && A.st->status) return;
-  __shared__ double red[2][TILE_T / 64];
-  const double rr = tile_sum_slots(A.pa + (size_t)par * 3 * A.G + A.G, A.G, red[0]);
-  const double bb = start ? tile_sum_slots(A.pa + 2 * A.G, A.G, red[1]) : A.st->bnorm2;
-  __syncthreads();
+// The test after the last iteration
+static __global__ __launch_bounds__(TILE_T) void k_tile_test(TileArgs A, int it) {
+  if (A.st->status) return;
+  __shared__ double red[TILE_T / 64];
+  const double rr = tile_sum_slots(A.pa + (size_t)(it & 1) * 3 * A.G + A.G, A.G, red);
   if (threadIdx.x == 0) {
-    const int it = start ? 0 : A.st->iters + 1;
-    const double tol2 = A.tol * A.tol;
-    A.st->bnorm2 = bb;
     A.st->rr = rr;
     A.st->iters = it;
-    A.st->status = (start && outer && *outer)                    ? 4
-                   : !(rr == rr && rr < INFINITY)                ? 2
-                   : ((start && bb == 0.0) || rr <= tol2 * bb)   ? 1
-                                                                 : (it >= A.maxiter ? 3 : 0);
+    A.st->status = tile_status(A, rr, A.st->bnorm2, it);
   }
 }
 

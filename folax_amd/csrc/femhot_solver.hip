@@ -923,14 +923,24 @@ static int pcg_async_core(Ctx *c, bool node_blocked, const long long *row_ptr, c
     int rc = tile_dispatch<double>(c->ndpn, tp, [&](auto p, auto l, auto sc) -> int {
       constexpr int P = decltype(p)::value, LPN = decltype(l)::value, S = decltype(sc)::value;
       const dim3 g(tp.G), t(TILE_T);
+      // Workgroups that make 4 or 8 passes wait for memory as often, with at most two waves per SIMD: with one
+      // dof per node a workgroup per pass and a kernel for p.q are faster (us an iteration: quads 300 x 300
+      // 18.6 -> 15.6, hexahedra 38^3 21.5 -> 16.7, 48^3 25.2 -> 24.8), with two, whose passes hold four times
+      // the values, slower (quads 350 x 350 26.5 -> 28.8); one workgroup alone has too few passes to gain.
+      constexpr bool may_split = P == 1 && S >= 4;
+      [[maybe_unused]] const long long passes = (c->Nn * LPN + TILE_T - 1) / TILE_T;
       hipLaunchKernelGGL((k_tile_init<P, LPN, S>), g, t, 0, s, A, V);
-      hipLaunchKernelGGL(k_tile_test, dim3(1), t, 0, s, A, 0, 1, outer);
       for (int k = 0; k < iterations; ++k) {
-        const int par = k & 1;
-        hipLaunchKernelGGL((k_tile_spmv<P, LPN, S>), g, t, 0, s, A, V, par, k == 0 ? 1 : 0);
-        hipLaunchKernelGGL((k_tile_update<P, LPN, S>), g, t, 0, s, A, V, par);
-        hipLaunchKernelGGL(k_tile_test, dim3(1), t, 0, s, A, 1 - par, 0, (const int *)nullptr);
+        bool split = false;
+        if constexpr (may_split)
+          if ((split = tp.G > 1)) {
+            hipLaunchKernelGGL((k_tile_pass<P, LPN>), dim3((unsigned)passes), t, 0, s, A, V, k, outer);
+            hipLaunchKernelGGL((k_tile_dot<P, LPN, S>), g, t, 0, s, A, V, k & 1);
+          }
+        if (!split) hipLaunchKernelGGL((k_tile_spmv<P, LPN, S>), g, t, 0, s, A, V, k, outer);
+        hipLaunchKernelGGL((k_tile_update<P, LPN, S>), g, t, 0, s, A, V, k & 1);
       }
+      hipLaunchKernelGGL(k_tile_test, dim3(1), t, 0, s, A, iterations);
       hipLaunchKernelGGL(k_pcg_finish, dim3(1), dim3(64), 0, s, A.st, iters, rel_res, status);
       FH_HIP(hipGetLastError());
       return FEMHOT_OK;
