@@ -148,6 +148,10 @@ class FiniteElementLoss:
             self.ctx.autotune(op, params, dofs, w, flags=self._flags() & ~L.SCATTER_CHUNK)
             self._tuned.add(key)
 
+    def _has_own(self, name):
+        """Whether a subclass, or this object, replaces a method of this class."""
+        return getattr(getattr(self, name), "__func__", None) is not getattr(FiniteElementLoss, name)
+
     def _one_call(self, bp, bd):
         """Whether a batch loss runs through its one-call entry points: device tensors of one floating type, the
         base class's dof and parameter vectors, and the Dirichlet values that the context holds."""
@@ -155,11 +159,8 @@ class FiniteElementLoss:
                 and bd.is_cuda and bp.device == bd.device and bp.dtype == bd.dtype
                 and bd.dtype in (torch.float32, torch.float64) and bp.dim() == 2 and bd.dim() == 2):
             return False
-        base = FiniteElementLoss
-        for name in ("GetFullDofVector", "GetParametersVectors"):  # a subclass's (or an object's) own
-            if getattr(getattr(self, name), "__func__", None) is not getattr(base, name):
-                return False
-        if self.get_param_function is not base._given_params:
+        if self._has_own("GetFullDofVector") or self._has_own("GetParametersVectors") \
+                or self.get_param_function is not FiniteElementLoss._given_params:
             return False
         self._dir_idx(bd.device)
         return self._dir_in_ctx

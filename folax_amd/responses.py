@@ -189,6 +189,9 @@ class FiniteElementResponse:
         d, u = self._inputs(nodal_control_values, nodal_dof_values)
         lam = _as_device_tensor(nodal_adj_dof_values, dtype=u.dtype, device=u.device).reshape(-1)
         q_d = self._point_grad(d, u, 0)
+        if self.fe_loss._has_own("ComputeResidualVJP"):
+            _, gk = self.fe_loss.ComputeResidualVJP(d, u, lam)
+            return self.fe_loss.ctx.gauss_point_gather(q_d.unsqueeze(0), self.fe_loss.num_gp).reshape(-1) + gk
         _, gk = self.fe_loss.ctx.residual_vjp(d.reshape(1, -1), u.reshape(1, -1), lam.reshape(1, -1), want_gu=False,
                                               flags=self.fe_loss._flags())
         if gk.numel() != self.fe_loss.ctx.n_nodes:  # an element field: the two have no common length
@@ -205,7 +208,8 @@ class FiniteElementResponse:
         wphi = (wdet * self.response_function(gp_d, gp_u)).contiguous()
         if wphi.shape != wdet.shape:
             raise RuntimeError(f"the response formula must give one value per Gauss point, got {tuple(wphi.shape)}")
-        if wphi.requires_grad:  # the caller differentiates the integrand's part
+        # the caller differentiates the integrand's part, or the loss has its own residual term
+        if wphi.requires_grad or self.fe_loss._has_own("ComputeResidualShapeVJP"):
             _, _, dndx = self._geometry(u.dtype, u.device)
             ge = torch.einsum("eg,egaj->eaj", wphi, dndx)                # (Ne, n, dim)
             if ge.shape[-1] < 3:
