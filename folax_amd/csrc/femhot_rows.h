@@ -55,6 +55,10 @@ __device__ __forceinline__ void shape_node(int a, double x, double y, double z, 
   }
 }
 
+// Whether the lanes of an element form the moments of its coordinates together: HEX8 beyond the one-point rule, whose
+// only Gauss-point lane needs three of the seven (30^3 thermal FP32 tangent: 24.8 us together, 22.7 alone).
+template <int ET, int NGP> constexpr bool rows_moments() { return ET == HEX8 && NGP > 1; }
+
 // Inverse Jacobian of Gauss point g of one element for the row-owner staging, with the shape function
 // values there: the arithmetic of gp_geometry (coordinates relative to node 0, J = sum_a x_a (x)
 // dN_a/dxi, inverse by cofactors), returning wdetJ.  xs: the element's node coordinates (N x 3, FP64).
@@ -66,16 +70,24 @@ __device__ __forceinline__ R gp_inverse(int g, const double *xs, R (&Nv)[ElemT<E
   constexpr int N = ElemT<ET>::N, D = ElemT<ET>::D;
   double xi, eta, zeta, w;
   gauss_point<ET, NGP>(g, xi, eta, zeta, w);
-  if constexpr (ET == HEX8) {  // xs holds the coordinates' moments (hex8_lane_moment)
+  if constexpr (ET == HEX8) {  // xs holds the coordinates' moments (rows_moments) or the coordinates
     R J[3][3];  // 8 J
     const R X = R(xi), Y = R(eta), Z = R(zeta), XY = R(xi * eta), XZ = R(xi * zeta), YZ = R(eta * zeta);
     constexpr int lane_of[8] = {0, 1, 3, 4, 2, 5, 7, 6};  // the lane that holds moment m
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       R m[8];
-      m[0] = R(0);
+      if constexpr (rows_moments<ET, NGP>()) {
+        m[0] = R(0);
 #pragma unroll
-      for (int k = 1; k < 8; ++k) m[k] = R(xs[lane_of[k] * 3 + i]);
+        for (int k = 1; k < 8; ++k) m[k] = R(xs[lane_of[k] * 3 + i]);
+      } else {
+        R col[8];
+        col[0] = R(0);
+#pragma unroll
+        for (int a = 1; a < 8; ++a) col[a] = R(xs[a * 3 + i] - xs[i]);
+        hex8_moments<R>(col, m);
+      }
       hex8_dxi<R>(m, X, Y, Z, XY, XZ, YZ, J[i]);
     }
 #pragma unroll
@@ -244,7 +256,10 @@ __device__ __forceinline__ void rows_column_starts(int lane, int kw, const unsig
 // Output stage: a lane owns row oc, component od and column kk of each round's CPW, and adds the column's
 // blocks in lane order.  The first four blocks of every round are loaded together, so their LDS latency is
 // paid once and not once a round (S reaches 3 blocks past the last); the sums stop at the column's end
-// by branches, for a select costs three instructions an entry.
+// by branches, for a select costs three instructions an entry.  With two dofs per node rounds past the node's
+// columns are left out: a window has four, and the 9 neighbours of a quadrilateral's node fill one (600 x 600 elastic
+// FP64 tangent: 302.6 us with their loads, 293.5 without; hexahedra fill all four of theirs, and
+// the test costs their 64^3 call 392 us against 385).
 template <class R, int N> __device__ __forceinline__ R rows_sum_four(int n, const R (&x)[N], R sum) {
   if (n > 0) {
     sum += x[0];
@@ -276,11 +291,14 @@ __device__ __forceinline__ void rows_add_columns(int kw, int oc, int kk, int od,
     n[r] = own ? CS[k + 1] - lo[r] : 0;
   }
 #pragma unroll
-  for (int r = 0; r < OR; ++r)
+  for (int r = 0; r < OR; ++r) {
+    if (P == 2 && r * CPW >= kw) continue;
 #pragma unroll
     for (int q = 0; q < 4; ++q) x[r][q] = S[(lo[r] + q) * (P * P) + oc * P + od];
+  }
 #pragma unroll
   for (int r = 0; r < OR; ++r) {
+    if (P == 2 && r * CPW >= kw) continue;
     R sum = rows_sum_four(n[r], x[r], R(0));
     for (int i = 4; i < n[r]; i += 4) {
       R y[4];
@@ -438,7 +456,7 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
         }
       }
 #pragma unroll
-      for (int i = 0; i < 3; ++i) XS[lane * 3 + i] = ET == HEX8 ? hex8_lane_moment(xc[i], b2) : xc[i];
+      for (int i = 0; i < 3; ++i) XS[lane * 3 + i] = rows_moments<ET, NGP>() ? hex8_lane_moment(xc[i], b2) : xc[i];
       for (int t = lane; t < kw; t += 64) MK[t] = 0ull;
       __syncthreads();
       // the lanes of each column of the window, as a bit mask
