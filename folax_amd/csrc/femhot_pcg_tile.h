@@ -592,14 +592,17 @@ __device__ __forceinline__ int tile_status(const TileArgs &A, double rr, double 
 }
 
 // Opens iteration k: every workgroup makes the test that precedes it (workgroup 0 records it; a workgroup that finds
-// its record already there reads the decision it would make) and takes beta.  False: the solve has ended.  A
-// kernel of its own for the test cost 2-3 us an iteration.
+// its record already there reads the decision it would make) and takes beta.  False: the solve has ended, for the
+// whole workgroup: one thread reads the record, which may change between two waves' reads.  A kernel of its own for
+// the test cost 2-3 us an iteration.
 __device__ __forceinline__ bool tile_open(const TileArgs &A, int k, const int *outer, double (*red)[TILE_T / 64],
                                           double &beta) {
-  if (k > 0 && A.st->status) return false;
+  __shared__ int ended;
+  if (threadIdx.x == 0) ended = k > 0 ? A.st->status : 0;
   const int par = k & 1;
   const double *now = A.pa + (size_t)par * 3 * A.G, *before = A.pa + (size_t)(1 - par) * 3 * A.G;
-  const double rr = tile_sum_slots(now + A.G, A.G, red[0]);
+  const double rr = tile_sum_slots(now + A.G, A.G, red[0]);  // (its barrier shows `ended` to all)
+  if (ended) return false;
   const double bb = k == 0 ? tile_sum_slots(now + 2 * A.G, A.G, red[1]) : A.st->bnorm2;
   const int status = k == 0 && outer && *outer ? 4 : tile_status(A, rr, bb, k);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
