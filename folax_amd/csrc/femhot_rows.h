@@ -24,8 +24,10 @@
 // FEMHOT_TRANSPOSE leaves them unchanged.
 //
 // Residual (A.R): formed in the same pass from the blocks, so a call that wants both reads the mesh and the
-// fields once and needs no second kernel, workspace or plan (HEX8 64^3 FP64, linear elastic: 495 us with the
-// residual through the chunk kernel, 447 here; 20^3: 47.9 and 37.8).
+// fields once and needs no second kernel, workspace or plan.  Linear elastic in FP64, with the residual through the chunk
+// kernel and here: tetrahedra 40^3 x 6 158 and 140 us, quads 200 x 200 46 and 38.  On elastic quads the gather of u and the
+// store of the residual cost a sixth of the tangent at every size, so from about 500 x 500 the separate kernel would be
+// faster once its plan is built (700 x 700: 433 and 447).
 #pragma once
 #include "femhot_kernels.h"
 
@@ -256,10 +258,11 @@ __device__ __forceinline__ void rows_column_starts(int lane, int kw, const unsig
 // Output stage: a lane owns row oc, component od and column kk of each round's CPW, and adds the column's
 // blocks in lane order.  The first four blocks of every round are loaded together, so their LDS latency is
 // paid once and not once a round (S reaches 3 blocks past the last); the sums stop at the column's end
-// by branches, for a select costs three instructions an entry.  With two dofs per node rounds past the node's
-// columns are left out: a window has four, and the 9 neighbours of a quadrilateral's node fill one (600 x 600 elastic
-// FP64 tangent: 302.6 us with their loads, 293.5 without; hexahedra fill all four of theirs, and
-// the test costs their 64^3 call 392 us against 385).
+// by branches, for a select costs three instructions an entry.  With two dofs per node the rounds go one at a time and
+// those past the node's columns are left out: a window has four, and the 9 neighbours of a quadrilateral's node fill one,
+// so loads for all four cost instructions and registers alone (300 x 300 elastic one-point tangent: FP64 54.0 us with 94
+// VGPRs, 48.5 with 78 and six waves per SIMD; FP32 41.0 and 35.5.  Hexahedra fill all four of theirs, and the test
+// costs their 64^3 call 392 us against 385).
 template <class R, int N> __device__ __forceinline__ R rows_sum_four(int n, const R (&x)[N], R sum) {
   if (n > 0) {
     sum += x[0];
@@ -281,32 +284,34 @@ template <class R, int N> __device__ __forceinline__ R rows_sum_four(int n, cons
 template <class R, int P, int CPW, int OR>
 __device__ __forceinline__ void rows_add_columns(int kw, int oc, int kk, int od, const R *S, const int *CS,
                                                  R (&acc)[OR]) {
-  int lo[OR], n[OR];
-  R x[OR][4];
+  constexpr int T = P == 2 ? 1 : OR;  // rounds whose loads are issued together
 #pragma unroll
-  for (int r = 0; r < OR; ++r) {
-    const int k = r * CPW + kk;
-    const bool own = k < kw && oc < P;
-    lo[r] = own ? CS[k] : 0;
-    n[r] = own ? CS[k + 1] - lo[r] : 0;
-  }
+  for (int r0 = 0; r0 < OR; r0 += T) {
+    if (P == 2 && r0 * CPW >= kw) continue;
+    int lo[T], n[T];
+    R x[T][4];
 #pragma unroll
-  for (int r = 0; r < OR; ++r) {
-    if (P == 2 && r * CPW >= kw) continue;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) x[r][q] = S[(lo[r] + q) * (P * P) + oc * P + od];
-  }
-#pragma unroll
-  for (int r = 0; r < OR; ++r) {
-    if (P == 2 && r * CPW >= kw) continue;
-    R sum = rows_sum_four(n[r], x[r], R(0));
-    for (int i = 4; i < n[r]; i += 4) {
-      R y[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) y[q] = S[(lo[r] + i + q) * (P * P) + oc * P + od];
-      sum = rows_sum_four(n[r] - i, y, sum);
+    for (int r = 0; r < T; ++r) {
+      const int k = (r0 + r) * CPW + kk;
+      const bool own = k < kw && oc < P;
+      lo[r] = own ? CS[k] : 0;
+      n[r] = own ? CS[k + 1] - lo[r] : 0;
     }
-    acc[r] += sum;
+#pragma unroll
+    for (int r = 0; r < T; ++r)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[r][q] = S[(lo[r] + q) * (P * P) + oc * P + od];
+#pragma unroll
+    for (int r = 0; r < T; ++r) {
+      R sum = rows_sum_four(n[r], x[r], R(0));
+      for (int i = 4; i < n[r]; i += 4) {
+        R y[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[q] = S[(lo[r] + i + q) * (P * P) + oc * P + od];
+        sum = rows_sum_four(n[r] - i, y, sum);
+      }
+      acc[r0 + r] += sum;
+    }
   }
 }
 template <class R, int P, int CPW, int OR>
@@ -314,6 +319,7 @@ __device__ __forceinline__ void rows_write(int kw, int k0, int deg, int oc, int 
                                            const R (&acc)[OR], R *V) {
 #pragma unroll
   for (int r = 0; r < OR; ++r) {
+    if (P == 2 && r * CPW >= kw) continue;  // (as rows_add_columns)
     const int k = r * CPW + kk;
     if (k >= kw || oc >= P) continue;
     R *v = V + oc * P * deg + (k0 + k) * P + od;
@@ -327,20 +333,50 @@ __device__ __forceinline__ R rows_apply(int kw, int oc, int kk, int od, const R 
   R s = R(0);
 #pragma unroll
   for (int r = 0; r < OR; ++r) {
+    if (P == 2 && r * CPW >= kw) continue;  // (as rows_add_columns)
     const int k = r * CPW + kk;
     if (k < kw && oc < P) s += acc[r] * DU[k * P + od];
   }
   return s;
 }
 
+// v of lane l (the same in all lanes) in all lanes.
+__device__ __forceinline__ float rows_lane(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double rows_lane(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// Sums over lanes 0..31 and 32..63, valid in lanes 31 and 63 (wave_sum_to_last without its last step).
+__device__ __forceinline__ float rows_from_15(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xa, 0xf, false));
+}
+__device__ __forceinline__ double rows_from_15(double v) { return dpp_f64<0x142, 0xa>(v); }
+template <class R> __device__ __forceinline__ R rows_half_sums(R v) {
+  v += lane_dpp<0xB1>(v);
+  v += lane_dpp<0x4E>(v);
+  v += lane_dpp<0x141>(v);
+  v += lane_dpp<0x140>(v);
+  return v + rows_from_15(v);
+}
+
 // The owned node's residual, masked as fe_loss.py:191-207: the output lanes' shares of K (u - u_i) (SHARES;
-// lane / G is the component) and, with lanes, each lane's own res, summed in a fixed order.  S: 64 values of scratch.
+// lane / G is the component) and, with lanes, each lane's own res, summed in a fixed order.  S: 64 values of scratch;
+// with one or two components those of each are the wave or a half of it, and register moves do (tangent and residual, 300 x
+// 300 quads, through scratch and by moves: thermal FP32 49.3 and 43.5 us, FP64 89.9 and 83.2, elastic FP32 62.2 and 59.9).
 template <class R, int P, int G, bool SHARES>
 __device__ __forceinline__ void rows_write_residual(R share, const R (&res)[P], bool lanes, unsigned dm,
                                                     bool accumulate, R *S, R *out) {
-  const int lane = threadIdx.x, c = lane >> 4;  // 16 lanes per component
+  constexpr int LPC = P == 1 ? 64 : P == 2 ? 32 : 16;  // lanes per component
+  static_assert(P == 3 || !SHARES || G == LPC, "a component's shares fill its lanes");
+  const int lane = threadIdx.x, c = lane / LPC;
+  const bool writer = (lane & (LPC - 1)) == LPC - 1 && c < P;
   R x = R(0);
-  if constexpr (SHARES) {
+  if constexpr (SHARES && P == 1) {
+    x = wave_sum_to_last(share);
+  } else if constexpr (SHARES && P == 2) {
+    x = rows_half_sums(share);
+  } else if constexpr (SHARES) {
     S[lane] = share;
     __syncthreads();
     for (int m = lane & 15; c < P && m < G; m += 16) x += S[c * G + m];
@@ -348,17 +384,16 @@ __device__ __forceinline__ void rows_write_residual(R share, const R (&res)[P], 
     x += lane_dpp<0x4E>(x);
     x += lane_dpp<0x141>(x);
     x += lane_dpp<0x140>(x);
-    __syncthreads();
   }
   const bool masked = (dm >> c) & 1;
   if (lanes) {
 #pragma unroll
     for (int k = 0; k < P; ++k) {
-      const R s = __shfl(wave_sum_to_last(res[k]), 63);
+      const R s = rows_lane(wave_sum_to_last(res[k]), 63);
       x += c == k ? s : R(0);
     }
   }
-  if ((lane & 15) == 0 && c < P) {
+  if (writer) {
     if (!accumulate)
       out[c] = masked ? R(0) : x;
     else if (!masked)
@@ -366,12 +401,16 @@ __device__ __forceinline__ void rows_write_residual(R share, const R (&res)[P], 
   }
 }
 
-// Waves per SIMD the compiler must fit: 3 for linear elasticity (168 VGPRs in FP64 HEX8 2x2x2, no spills);
-// the thermal instantiations keep the compiler's own choice (the powc of k(T) would spill under 3).
-template <int PH> constexpr int rows_min_waves() { return PH == MECH ? 3 : 1; }
+// Waves per SIMD the compiler must fit: 3 for linear elasticity (130 VGPRs at most, at the 27-point rule of HEX8, no spills);
+// the thermal instantiations keep the compiler's own choice (the powc of k(T) would spill), except that FP64 tetrahedra at
+// four points, whose choice is 3, take 4 with 4 spilled registers (24^3 x 6, tangent: 32.0 us at 3 waves, 29.5 at 4).
+template <class R, int ET, int PH, int NGP> constexpr int rows_min_waves() {
+  if (PH == MECH) return 3;
+  return ET == TET4 && NGP == 2 && sizeof(R) == 8 ? 4 : 1;
+}
 
 template <class R, int ET, int PH, int NGP>
-__global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs A) {
+__global__ __launch_bounds__(64, (rows_min_waves<R, ET, PH, NGP>())) void k_tangent_rows(TArgs A) {
   static_assert(PH != NEOHOOKE, "row-owner assembly covers thermal and linear elasticity");
   using E = Elem<R, ET, PH>;
   constexpr int N = E::N, D = E::D, P = E::P;
@@ -580,12 +619,12 @@ __global__ __launch_bounds__(64, rows_min_waves<PH>()) void k_tangent_rows(TArgs
       rows_add_columns<R, P, CPW, OR>(kw, oc, kk, od, S, CS, acc);  // 3. each output sums its column's blocks
       __syncthreads();  // before the next batch overwrites the blocks and the masks
     }
-    rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
-    if (want_r) share += rows_apply<R, P, CPW, OR>(kw, oc, kk, od, DU, acc);
+    if (want_r) (P == 1 ? res[0] : share) += rows_apply<R, P, CPW, OR>(kw, oc, kk, od, DU, acc);
     __syncthreads();  // before the next window's DU
+    rows_write<R, P, CPW, OR>(kw, k0, deg, oc, kk, od, accumulate, acc, V);
   }
-  if (want_r)
-    rows_write_residual<R, P, CPW * P, true>(share, res, A.pp.has_body, (unsigned)__ballot(dmv != 0), accumulate, S,
+  if (want_r)  // (one dof per node: every lane's share and body force in one sum over the wave)
+    rows_write_residual<R, P, CPW * P, P != 1>(share, res, P == 1 || A.pp.has_body, (unsigned)__ballot(dmv != 0), accumulate, S,
                                              reinterpret_cast<R *>(A.R) + node * P);
 }
 

@@ -63,9 +63,10 @@ template <class R> __device__ __forceinline__ R hex8_node_sum(R q0, R q1, R q2) 
   return (w0 + g * hex8_across<2>(w0)) + (w2 - hex8_across<2>(w2));
 }
 
-// Waves per SIMD the compiler must fit, by measurement at 64^3 (us with the residual): thermal FP64 272 at 4 waves, 315
-// at 3, 433 at 5 (the general power of k(T) spills); thermal FP32 141 at 8, 149 at 7; linear elastic FP64 5 (4: 450,
-// 6: 700), FP32 4 or more alike (270); Neo-Hookean FP64 1211 at 2, 1650 at 1, FP32 4 or 5 alike (585).
+// Waves per SIMD the compiler must fit, by measurement at 64^3 (us with the residual): thermal FP64 272 at 4 waves (2
+// spilled registers), 315 at 3 (none), 433 at 5 (the general power of k(T) spills more); thermal FP32 141 at 8, 149 at 7;
+// linear elastic FP64 5 (4: 450, 6: 700), FP32 4 or more alike (270); Neo-Hookean FP64 1211 at 2 (7 spilled), 1650 at 1,
+// FP32 4 or 5 alike (585).
 template <class R, int PH> constexpr int rows_hex8_waves() {
   if (sizeof(R) == 4) return PH == THERMAL ? 8 : 4;
   return PH == NEOHOOKE ? 2 : PH == THERMAL ? 4 : 5;
