@@ -41,10 +41,12 @@ __device__ __forceinline__ double sum_partials(const double *part) {
 
 // Both SpMV kernels take `rev`: the workgroups then walk the tiles from the last to the first.  Consecutive
 // iterations alternate, so a sweep starts on the part of the matrix that the sweep before left in the
-// 256 MB memory-side cache, where a forward sweep each time finds its beginning gone (matrices up to that
-// size stay cached either way): HEX8 64^3, 518 MB of FP64 values, 157 -> 146 us per iteration, 259 MB of
-// FP32 values 96 -> 85; 52^3 FP64, 279 MB, 87 -> 78; 40^3, 127 MB, 41.7 both ways.  Partials are stored by
-// tile, so the sums, and the iterates, are the same.
+// 256 MB memory-side cache, where a forward sweep each time finds its beginning gone.  An iteration, always forward
+// -> alternating: HEX8 64^3, 518 MB of FP64 values, 158.7 -> 147.1 us, 259 MB of FP32 values 97.9 -> 87.6; 52^3 FP64,
+// 281 MB, 88.4 -> 79.0; 40^3, 127 MB, 42.0 both ways.  A matrix that the L2 caches hold together is always walked forward:
+// turned round, a tile comes to another XCD, whose L2 has not seen it (any-pattern solve, HEX8 20^3 elastic, 24 MB
+// with its columns, 20.1 -> 21.1; thermal 40^3, 22 MB, 21.1 -> 22.2; 42 MB 25.0 both ways).  Partials are stored by tile, so
+// the sums, and the iterates, are the same.
 //
 // y = A x, LPR lanes per row, one pass (grid = rows * LPR / 256).  Each lane first loads up to U = 8
 // of its row's (column, value) pairs, then gathers x for all of them, so a row costs three dependent
@@ -317,6 +319,9 @@ static SpmvPlan spmv_plan(long long n, long long nnz, int P, bool node_blocked) 
   return sp;
 }
 
+// Whether consecutive sweeps of a matrix of T alternate: values and columns beyond the 8 L2 caches of 4 MB.
+template <class T> static bool spmv_alternates(long long nnz) { return nnz * (long long)(sizeof(T) + sizeof(int)) > (32LL << 20); }
+
 template <class T, int P>
 static void spmv_node_launch(long long nodes, const long long *rp, const int *ci, const T *v, const T *x, T *y,
                              double *part, const SpmvPlan &sp, hipStream_t s, const int *stop, int rev) {
@@ -378,9 +383,10 @@ static int pcg_core(Ctx *c, long long n, const long long *rp, const int *ci, con
     return FEMHOT_OK;
   }
   int k = 0;
+  const bool alt = spmv_alternates<T>(c->nnz);
   while (k < maxiter) {
     const int par = k & 1;
-    spmv_launch<T>(n, rp, ci, v, p, q, pap_part, sp, s, nullptr, par);
+    spmv_launch<T>(n, rp, ci, v, p, q, pap_part, sp, s, nullptr, alt ? par : 0);
     hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, s, pap_part, (long long)nsp, pap, (const int *)nullptr);
     hipLaunchKernelGGL((k_update_xr<T>), grid, dim3(256), 0, s, n, x, r, p, q, dinv, rz[par], pap, rz[1 - par], rrp,
                        (const int *)nullptr);
@@ -967,9 +973,10 @@ static int pcg_async_core(Ctx *c, bool node_blocked, const long long *row_ptr, c
   spmv_launch<double>(n, row_ptr, col_idx, vals, x, r, nullptr, sp, s);  // r = A x
   hipLaunchKernelGGL((k_init<double>), nbr, dim3(256), 0, s, n, b, r, p, dinv, rz[0], rrp);
   hipLaunchKernelGGL(k_pcg_start, dim3(1), dim3(1024), 0, s, aux, rrp, tol2, iterations, outer, st);
+  const bool alt = spmv_alternates<double>(c->nnz);
   for (int k = 0; k < iterations; ++k) {  // the same kernels as femhot_pcg; a stopped solve skips them
     const int par = k & 1;
-    spmv_launch<double>(n, row_ptr, col_idx, vals, p, q, pap_part, sp, s, stop, par);
+    spmv_launch<double>(n, row_ptr, col_idx, vals, p, q, pap_part, sp, s, stop, alt ? par : 0);
     hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, s, pap_part, (long long)nsp, pap, stop);
     hipLaunchKernelGGL((k_update_xr<double>), nbr, dim3(256), 0, s, n, x, r, p, q, dinv, rz[par], pap, rz[1 - par],
                        rrp, stop);
