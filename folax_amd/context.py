@@ -131,6 +131,20 @@ class FemhotContext:
             raise ValueError(f"{name} must be contiguous in its last dimension")
         return t.stride(0) if batch > 1 else last
 
+    @staticmethod
+    def _check_vector(t, name, size, dtype, device):
+        """_check_in for one sample's contiguous vector."""
+        if not t.is_cuda:
+            raise ValueError(f"{name} must be a device tensor")
+        if t.dtype != dtype:
+            raise TypeError(f"{name} has dtype {t.dtype}, expected {dtype}")
+        if t.device != device:
+            raise ValueError(f"{name} is on {t.device}, expected {device}")
+        if t.numel() != size:
+            raise ValueError(f"{name} must have shape (1, {size}), got (1, {t.numel()})")
+        if not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous in its last dimension")
+
     def _field_size(self, flags):
         return self.n_elems if flags & L.ELEMENT_FIELD else self.n_nodes
 
@@ -248,16 +262,16 @@ class FemhotContext:
         u, w = u.reshape(-1), w.reshape(-1)
         field = field.reshape(-1)
         dt, dev = u.dtype, u.device
-        self._check_in(u.view(1, -1), "u", self.n_dofs, 1, dt, dev)
-        self._check_in(w.view(1, -1), "w", self.n_dofs, 1, dt, dev)
-        self._check_in(field.view(1, -1), "field", self._field_size(flags), 1, dt, dev)
-        gx = torch.empty(self.n_nodes, 3, dtype=dt, device=dev)
+        self._check_vector(u, "u", self.n_dofs, dt, dev)
+        self._check_vector(w, "w", self.n_dofs, dt, dev)
+        self._check_vector(field, "field", self._field_size(flags), dt, dev)
+        gx = u.new_empty((self.n_nodes, 3))
         dim = 2 if self.et == L.QUAD4 else 3
         if wphi is not None:
             G = self._points(self.num_gp)
             if wphi.dtype != dt or wphi.device != dev or not wphi.is_contiguous() or wphi.numel() != self.n_elems * G:
                 raise ValueError(f"wphi must be a contiguous ({self.n_elems}, {G}) tensor of u's dtype and device")
-        scratch = torch.empty(self.n_elems * self.nodes_per_elem * dim, dtype=dt, device=dev)
+        scratch = u.new_empty(self.n_elems * self.nodes_per_elem * dim)
         L.check(self._lib.femhot_shape_gradient(self._h, _dtype_code(u), _ptr(field), _ptr(u), _ptr(w), _ptr(wphi),
                                                 _ptr(scratch), _ptr(gx), flags, _stream()))
         return gx
