@@ -92,16 +92,6 @@ template <class R, int K> __device__ __forceinline__ void store_corner_results(R
   }
 }
 
-// LDS layout of k_chunk (in units of R unless noted; cap4 = max chunk nodes rounded up to 4,
-// emax = max chunk elements):
-//   X   [cap4 * 3]      chunk-relative coordinates (x, y, z)
-//   U   [cap4 * P]      nodal solution
-//   W   [cap4 * P]      cotangent (VJP only)
-//   FD  [cap4]          nodal field (nodal fields only)
-//   ER  [(emax * N + cap4 * pad) * P]  per element corner: residual / g_u, at [incidence-list position
-//                       (the plan's rank of the corner) + pad * chunk node][component], so each node's
-//                       corners are one contiguous run
-//   ERD [emax * N + cap4 * pad]  per element corner, at the same row: nodal field-gradient contribution
 // s += the P-vectors lo .. hi - 1 of E (LDS) in order.  Four are loaded before the first is added: one at a
 // time, a node's sum pays the LDS latency once per corner, the longest serial chain of the kernel (24 corners
 // for an interior node of a tetrahedral mesh).  The last, partial four re-read the last corner and add -0,
@@ -141,6 +131,16 @@ template <class R, int ET, int PH, int MODE, int BLOCK> constexpr int chunk_min_
   return (sizeof(R) == 4 && ET == TET4 && PH != NEOHOOKE && BLOCK == 256) ? 4 : 1;
 }
 
+// LDS layout of k_chunk (in units of R unless noted; cap4 = max chunk nodes rounded up to 4,
+// emax = max chunk elements):
+//   X   [cap4 * 3]      chunk-relative coordinates (x, y, z)
+//   U   [cap4 * P]      nodal solution
+//   W   [cap4 * P]      cotangent (VJP only)
+//   FD  [cap4]          nodal field (nodal fields only)
+//   ER  [(emax * N + cap4 * pad) * P]  per element corner: residual / g_u, at [incidence-list position
+//                       (the plan's rank of the corner) + pad * chunk node][component], so each node's
+//                       corners are one contiguous run
+//   ERD [emax * N + cap4 * pad]  per element corner, at the same row: nodal field-gradient contribution
 template <class R, int ET, int PH, int NGP, int MODE, int BLOCK>
 __global__ __launch_bounds__(BLOCK, (chunk_min_waves<R, ET, PH, MODE, BLOCK>())) void k_chunk(ChunkArgs A) {
   using E = Elem<R, ET, PH>;

@@ -202,7 +202,7 @@ template <class T, int P, int LPN, int S> struct Tile {
 // between XCDs), then the LDS gathers of the SpMV; the matrix is read once.  512 threads at 256 VGPRs
 // (one workgroup per CU) hold S x 4 blocks per lane; 1024 threads at 128 VGPRs spilled.  One iteration,
 // four launched kernels -> here: quads 40 x 40 conduction FP64 17 -> 4.0 us, hexahedra 17 x 13 x 11 elastic
-// FP64 18 -> 5.5 us, 43 x 37 x 29 mixed (its FP32 matrix, 46 MB, in 197 workgroups' registers) 22 -> 7.8 us.
+// FP64 18 -> 5.5 us, 43 x 37 x 29 mixed (its FP32 matrix, 46 MB, in 196 workgroups' registers) 22 -> 7.8 us.
 template <class T, int P, int LPN, int S>
 __global__ __launch_bounds__(TILE_T) void k_pcg_resident(TileArgs A) {
   using G_ = Tile<T, P, LPN, S>;
