@@ -41,16 +41,22 @@ class _ArrayNamespace:
 def _kernels_read(*tensors):
     """Whether the gather kernels can take these tensors: plain ones with memory of their own, outside torch's
     transforms (functorch, forward mode, batched gradients) and traces, which need operators they know."""
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter)
-                and not torch._C._functorch.is_functorch_wrapped_tensor(t) and _has_memory(t) for t in tensors)
-            and forward_ad._current_level < 0 and not torch._C._len_torch_dispatch_stack()
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+    if (forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() or torch._C._is_tracing()
+            or torch.compiler.is_compiling()):
+        return False
+    for t in tensors:
+        if not (type(t) in (torch.Tensor, torch.nn.Parameter) and _has_memory(t)) \
+                or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+    return True
 
 
 def _point_values(r, d, u):
     """N.d (n_elems, G) and N.u (dofs per node, n_elems, G) of response r's mesh: by the kernel, or by torch's own
     operators where that cannot be (the linear map is the same)."""
     if _kernels_read(d, u):
+        if not (torch.is_grad_enabled() and (d.requires_grad or u.requires_grad)):  # nothing to record
+            return r.fe_loss.ctx.gauss_point_values(d.contiguous(), u.contiguous(), r.fe_loss.num_gp)
         return _PointValues.apply(r, d, u)
     N, conn = r._geometry(u.dtype, u.device)[0], r._connectivity(u.device)
     return d[conn] @ N.T, u.view(-1, r.fe_loss.number_dofs_per_node)[conn].permute(2, 0, 1) @ N.T
