@@ -240,7 +240,7 @@ class FiniteElementLoss:
         bp = torch.atleast_2d(bp).reshape(bp.shape[0] if bp.dim() > 1 else 1, -1)
         bd = torch.atleast_2d(bd).reshape(bd.shape[0] if bd.dim() > 1 else 1, -1)
         if self.loss_function_exponent == 1.0 and self._one_call(bp, bd):
-            m, low, high = _BatchLoss.apply(self, bp, bd)
+            m, low, high, _ = _BatchLoss.apply(self, bp, bd)
             return m, (low, high, m)
         full = _FullDofs.apply(self, bp, bd)
         energies = _BatchEnergy.apply(self, torch.atleast_2d(self.GetParametersVectors(bp)), full)
@@ -315,9 +315,10 @@ class FiniteElementLoss:
 
 class _BatchLoss(torch.autograd.Function):
     """ComputeBatchLoss with exponent 1 in one library call per pass: (mean, min, max) of the samples'
-    energies.  The residual, which the forward kernel forms anyway, is the energies' gradient with
-    respect to the dofs (see _BatchEnergy), so the backward pass scales it; the control gradient, where
-    asked for, takes the kernels of _BatchEnergy."""
+    energies, and the energies, which stay inside.  The residual, which the forward kernel forms anyway, is the
+    energies' gradient with respect to the dofs (see _BatchEnergy), so the backward pass scales it; the control
+    gradient, where asked for, takes the kernels of _BatchEnergy.  Under create_graph the gradients keep the tie to
+    the energies that their power 1 has in the composed loss, whose second derivative is zero."""
 
     @staticmethod
     def forward(ctx, loss, params, dofs):
@@ -331,14 +332,14 @@ class _BatchLoss(torch.autograd.Function):
         keep_p = ctx.body or (need_p and loss.physics != L.MECHANICAL)
         ctx.save_for_backward(params if keep_p else None, full if keep_p else None, R, en)
         ctx.shape, ctx.dtype = params.shape, dofs.dtype
-        return mean, low, high
+        return mean, low, high, en
 
     @staticmethod
-    def backward(ctx, g, g_low, g_high):
+    def backward(ctx, g, g_low, g_high, g_en):
         loss = ctx.loss
         params, full, R, en = ctx.saved_tensors
         flags, batch = loss._flags(), en.shape[0]
-        plain = (g_low is None and g_high is None and not torch.is_grad_enabled()
+        plain = (g_low is None and g_high is None and g_en is None and not torch.is_grad_enabled()
                  and (g is None or _has_memory(g)))
         if plain and g is not None:
             g = g.contiguous()
@@ -350,6 +351,8 @@ class _BatchLoss(torch.autograd.Function):
                     at = extreme(e)
                     tie = ((e == at) | (e.isnan() & at.isnan())).to(e.dtype)
                     s = s + ge * tie / tie.sum()
+            if torch.is_grad_enabled():
+                s = s * e.pow(0.0)
             s = s.reshape(-1, 1)
         elif g is None:
             return None, None, None
@@ -370,7 +373,11 @@ class _BatchLoss(torch.autograd.Function):
                 _, _, gd = loss.ctx.energy_grad(params, full, want_gu=False, want_energy=False, flags=flags)
             elif loss.physics == L.THERMAL:
                 _, gd = loss.ctx.residual_vjp(params, full, full, want_gu=False, flags=flags)
-            gd = scaled(gd) if gd is not None else torch.zeros(ctx.shape, dtype=ctx.dtype, device=en.device)
+            if gd is None:  # linear elastic: none
+                gd = torch.zeros(ctx.shape, dtype=ctx.dtype, device=en.device)
+                gd = gd if plain else gd * s
+            else:
+                gd = scaled(gd)
         return None, gd, gu
 
 
