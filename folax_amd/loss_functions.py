@@ -237,8 +237,9 @@ class FiniteElementLoss:
         """fe_loss.py:250-262: mean_b (sum_e E_e)^p with (min, max, mean); differentiable."""
         bd = _as_device_tensor(batch_dofs) if not isinstance(batch_dofs, torch.Tensor) else batch_dofs
         bp = batch_params if isinstance(batch_params, torch.Tensor) else _as_device_tensor(batch_params, dtype=bd.dtype)
-        bp = torch.atleast_2d(bp).reshape(bp.shape[0] if bp.dim() > 1 else 1, -1)
-        bd = torch.atleast_2d(bd).reshape(bd.shape[0] if bd.dim() > 1 else 1, -1)
+        if not (bp.dim() == 2 and bd.dim() == 2 and bp.numel() and bd.numel()):
+            bp = torch.atleast_2d(bp).reshape(bp.shape[0] if bp.dim() > 1 else 1, -1)
+            bd = torch.atleast_2d(bd).reshape(bd.shape[0] if bd.dim() > 1 else 1, -1)
         if self.loss_function_exponent == 1.0 and self._one_call(bp, bd):
             m, low, high, _ = _BatchLoss.apply(self, bp, bd)
             return m, (low, high, m)
